@@ -324,6 +324,28 @@ int sf_tree_attention(const void *q, int64_t q_stride_token,
                       void *out, sf_stream_t stream);
 
 /*
+ * sf_tree_attention with scratch memory that lets a call of few query rows
+ * split its keys over the chip: each split's (max, sum, accumulator) goes to
+ * the workspace in fp32 and a second kernel merges them in split order.
+ * sf_tree_attention_workspace returns the bytes a call of that shape (masked:
+ * with a mask) can use (0: it would not split).  workspace: device memory, 16-byte aligned, in use
+ * until the call's kernels have run; with less than the needed bytes (or
+ * NULL) the call runs unsplit.  Results of the two forms differ by the order
+ * of the fp32 sums.
+ */
+int64_t sf_tree_attention_workspace(int queries, int keys, int q_heads,
+                                    int kv_heads, int head_dim, int masked);
+int sf_tree_attention_split(const void *q, int64_t q_stride_token,
+                            int64_t q_stride_head, const void *k,
+                            int64_t k_stride_head, int64_t k_stride_token,
+                            const void *v, int64_t v_stride_head,
+                            int64_t v_stride_token, const uint8_t *mask,
+                            int64_t mask_stride_query, int queries, int keys,
+                            int q_heads, int kv_heads, int head_dim,
+                            float scale, void *out, void *workspace,
+                            int64_t workspace_bytes, sf_stream_t stream);
+
+/*
  * K6: RMSNorm over the last dimension.  Replaces Qwen3MoeRMSNorm.forward
  * (tf:294-299):
  *   v = mean over d of float(x[r, d])^2 (fp32)

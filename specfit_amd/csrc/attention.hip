@@ -10,15 +10,17 @@
 // i.e. causal aligned to the end of the keys).  A query with no admitted key
 // gets 0.
 //
-// At verification sizes (Q = 61 tree tokens, S ~ 1.1k keys, 32 query heads,
-// 4 KV heads, head dim 128) the whole layer's K/V is ~2 MB: the kernel is
-// latency-bound, not HBM-bound.  Head dims 64 and 128 with 2..16 query heads
-// per KV head run the MFMA form below (26 us at the 61-token verification
-// shape and 28 us at 128 tokens on MI355X, against 54 and 108 us for the
-// loop form).  The loop form covers every other shape: one workgroup per
-// (query, KV head) keeps the
-// G query heads of the group together so each K/V row is read once per
-// query.  Its 8 wavefronts take interleaved 64-key chunks: scores with one
+// Head dims 64 and 128 with 2..16 query heads per KV head run the tiled MFMA
+// form below; measured on MI355X at 32 query / 4 KV heads of 128, against the
+// 16-row MFMA form it replaced: a 4096-token prompt 1562 -> 162 us (850
+// TFLOP/s of the causal half), one token over 4096 keys 49 -> 10 us of device
+// time, a 61-node tree over 1085 keys 26 -> 16 us.  What bounds it: prompts,
+// the softmax's vector work next to the matrix work (each SIMD has two
+// wavefronts, which overlap only in part); decoding and trees, latency (the
+// K/V of 1085 keys is 2 MB).
+// The loop form covers every other shape: one workgroup per (query, KV head)
+// keeps the G query heads of the group together so each K/V row is read once
+// per query.  Its 8 wavefronts take interleaved 64-key chunks: scores with one
 // key per lane (the key row in registers, the query rows broadcast from
 // LDS), an online softmax per head across the wavefront, then P.V with the
 // head-dim elements spread over the lanes and the value rows of 16 keys
@@ -276,267 +278,582 @@ __global__ __launch_bounds__(NW * SF_WAVE) void tree_attention_kernel(const Attn
   }
 }
 
-// ------------------------------------------------------- MFMA form --
+// ------------------------------------------------------ tiled MFMA form --
 // For head dims 64 / 128 and 2..16 query heads per KV head, with 16-byte
-// aligned rows.  A workgroup owns one KV head and a tile of 16 query rows
-// (16 / G tokens x the G heads of the group) and all keys; its 8 wavefronts
-// take interleaved 32-key chunks.  Per chunk a wavefront computes the
-// 16 x 32 score tile with v_mfma_f32_16x16x32_bf16 (A = query rows, B = key
-// rows: both 8 consecutive head-dim elements per lane, straight from
-// memory), applies the scale and the mask, updates its online softmax per
-// row (rows 4 (l / 16) + i of lane l, reduced over the 16 lanes that share
-// them), and adds P.V with P (bf16) read back from LDS as the A operand and
-// the chunk's value rows staged in LDS (B: 8 keys of one head-dim column per
-// lane).  The 8 wavefront states are merged in wavefront order, so the
-// result is run-to-run identical.
-constexpr int kMfmaWaves = 8;
-constexpr int kKeysPerChunk = 32;
-constexpr int kPRow = kKeysPerChunk * 2 + 16;  // P row in LDS (bytes, padded)
+// aligned rows.  The Q tokens x G heads of one KV head form R = Q G query
+// rows that share its keys and values.  A wavefront owns 32 of these rows
+// and walks the keys in tiles of 64; the four wavefronts of a workgroup are
+// WR row groups x 4 / WR key groups:
+//   WR = 4: 128 rows; each K/V tile is staged once for the four wavefronts
+//           (two LDS buffers, one barrier per tile; registers hold the next
+//           tile's loads).  The form of prompts.
+//   WR = 1: 32 rows; each wavefront takes every fourth tile into LDS of its
+//           own (no barrier until the states are merged).  The form of
+//           decoding and of small draft trees.
+// The keys are also split over workgroups when the row tiles alone would
+// leave the chip idle: each split writes its (max, sum, accumulator) in fp32
+// to the caller's workspace and combine_kernel merges them in split order.
+//
+// Scores are computed transposed, S^T = K Q^T (v_mfma_f32_32x32x16_bf16, A =
+// key rows, B = query rows): lane l then holds 32 of the tile's 64 scores of
+// query row l % 32 and lane l ^ 32 the other 32, so the softmax state is one
+// register per lane and its reductions are in-lane but for one half swap.
+// O^T += V^T P^T takes the probabilities (bf16) as the B operand straight
+// from those registers: the 16 keys of a k-step are {8 g + 4 (l / 32) ..+3},
+// g = 0, 1, on both sides, and the V^T fragments in that order come from
+// ds_read_b64_tr_b16 on the row-major value tile.
+typedef float sf_f32x16 __attribute__((ext_vector_type(16)));
+typedef short sf_i16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 sf_bf16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int sf_u32x4 __attribute__((ext_vector_type(4)));
 
-template <int D>
-constexpr int v_row_bytes() { return D * 2 + 8; }  // 8 B pad: the four 8-row groups hit distinct banks
+constexpr int kTileKeys = 64;
+constexpr int kTileWaves = 4;
+constexpr int kTileThreads = kTileWaves * SF_WAVE;
+constexpr int kMaxSplits = 64;
 
+struct TiledArgs {
+  AttnArgs a;
+  int log_g;         // G = 1 << log_g
+  int rows;          // Q * G
+  int row_tiles;     // of 32 WR rows
+  int splits;
+  int split_keys;    // keys of one split, a multiple of 64 * 4 / WR
+  float* part_acc;   // [splits][Hkv][rows][D], splits > 1 only
+  float2* part_ml;   // [splits][Hkv][rows] (max in log2 units, sum)
+};
+
+// Rows padded so the fragment reads spread over the banks: 16 B for the
+// 16-byte reads of K (16 consecutive rows), 32 B for the transposed reads of
+// V (32 B of each of 4 rows).
 template <int D>
-constexpr size_t mfma_lds_bytes() {
-  constexpr size_t loop = kMfmaWaves * (kKeysPerChunk * v_row_bytes<D>() + 16 * kPRow);
-  constexpr size_t merge = kMfmaWaves * 16 * (D + 2) * sizeof(float);
+struct TileLds {
+  static constexpr int krow = 2 * D + 16;
+  static constexpr int vrow = 2 * D + 32;
+  static constexpr int bytes = kTileKeys * (krow + vrow);
+  static constexpr int orow = D + 4;  // floats, merge of the key groups
+};
+
+template <int D, int WR>
+constexpr int tiled_lds_bytes() {
+  constexpr int loop = (WR == 4 ? 2 : 4 / WR) * TileLds<D>::bytes;
+  constexpr int merge = WR == 4 ? 0 : (4 / WR) * 32 * WR * (TileLds<D>::orow + 2) * 4;
   return loop > merge ? loop : merge;
 }
 
-__device__ __forceinline__ sf_f32x4 mfma_bf16(uint4 a, uint4 b, sf_f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sf_bf16x8, a),
-                                                 __builtin_bit_cast(sf_bf16x8, b), c, 0, 0, 0);
+__device__ __forceinline__ sf_f32x16 mfma_32(sf_bf16x8 a, sf_bf16x8 b, sf_f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// Max / sum over the 16 lanes of a lane's row group (lanes 16 g .. 16 g + 15,
-// one DPP row): the group_sum moves, with max for the max.
-template <int CTRL>
-__device__ __forceinline__ float dpp_max(float x) {
-  const int moved = __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false);
-  return fmaxf(x, __int_as_float(moved));
+// 16-byte load, explicitly from global memory (a flat load would also hold
+// up the LDS waits).  With a byte offset: uniform address + 32-bit offset.
+__device__ __forceinline__ sf_u32x4 ld16(const uint16_t* p) {
+  return *(const __attribute__((address_space(1))) sf_u32x4*)(p);
 }
 
-__device__ __forceinline__ float row16_max(float x) {
-  x = dpp_max<0xB1>(x);
-  x = dpp_max<0x4E>(x);
-  x = dpp_max<0x141>(x);
-  return dpp_max<0x140>(x);
+__device__ __forceinline__ sf_u32x4 ld16(const uint16_t* p, uint32_t byte_offset) {
+  return *(const __attribute__((address_space(1))) sf_u32x4*)(reinterpret_cast<const char*>(p) + byte_offset);
 }
 
-__device__ __forceinline__ float row16_sum(float x) { return group_sum<16>(x); }
+// max(x, y) as one instruction: fmaxf first canonicalises operands that come
+// from a matrix instruction.  A NaN operand gives the other one, as fmaxf.
+__device__ __forceinline__ float max_raw(float x, float y) {
+  return __builtin_amdgcn_fmed3f(x, y, INFINITY);
+}
 
-template <int G, int D>
-__global__ __launch_bounds__(kMfmaWaves * SF_WAVE) void tree_attention_mfma_kernel(
-    const AttnArgs a) {
-  constexpr int kTok = 16 / G;        // tokens per 16-row tile
-  constexpr int kSteps = D / 32;      // MFMA k-steps of a score tile
-  constexpr int kNt = D / 16;         // 16-wide head-dim tiles of the output
-  constexpr int kVRow = v_row_bytes<D>();
-  __shared__ __attribute__((aligned(16))) char lds[mfma_lds_bytes<D>()];
+// Four values of a column of a row-major bf16 tile: the 16 lanes of a group
+// pass the addresses of 4 rows x 4 eight-byte pieces, lane i gets column i.
+__device__ __forceinline__ sf_i16x4 read_tr4(const char* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) sf_i16x4*)(p));
+}
+
+// Value of the lane 32 away combined with the own one.
+__device__ __forceinline__ float half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
+  return fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
+}
+
+__device__ __forceinline__ float half_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
+  return __int_as_float(r[0]) + __int_as_float(r[1]);
+}
+
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  const sf_bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
+  return __builtin_bit_cast(uint32_t, v);
+}
+
+// Mask bytes of keys key .. key + 3 of one row (0 past the last key).
+__device__ __forceinline__ uint32_t mask_word(const uint8_t* row, int key, int S) {
+  uint32_t w = 0;
+  if (key + 4 <= S) {
+    __builtin_memcpy(&w, row + key, 4);
+  } else {
+    for (int i = 0; key + i < S; ++i) w |= static_cast<uint32_t>(row[key + i]) << (8 * i);
+  }
+  return w;
+}
+
+// One more (max, sum, accumulator) state, weighted against the maximum M.
+__device__ __forceinline__ void add_state(float m, float l, const float4& v, float M, float& sum,
+                                          float (&o)[4]) {
+  const float f = __builtin_amdgcn_exp2f(m - M);
+  sum = __builtin_fmaf(l, f, sum);
+  o[0] = __builtin_fmaf(v.x, f, o[0]);
+  o[1] = __builtin_fmaf(v.y, f, o[1]);
+  o[2] = __builtin_fmaf(v.z, f, o[2]);
+  o[3] = __builtin_fmaf(v.w, f, o[3]);
+}
+
+// Elements d .. d + 3 of query row r (token r / G) of KV head h, divided by
+// the row's sum (0 where the row admits no key).
+__device__ __forceinline__ void store_row4(const TiledArgs& t, int h, int r, int D, int d,
+                                           const float (&o)[4], float sum) {
+  const int64_t hq = static_cast<int64_t>(t.a.Hkv) << t.log_g;
+  const int64_t head = (static_cast<int64_t>(h) << t.log_g) + (r & ((1 << t.log_g) - 1));
+  const float inv = 1.f / sum;
+  float y[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = sum > 0.f ? o[i] * inv : 0.f;
+  *reinterpret_cast<uint2*>(t.a.out + ((r >> t.log_g) * hq + head) * D + d) =
+      make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
+}
+
+template <int D, int WR, bool MASK>
+__global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_tiled_kernel(
+    const TiledArgs t) {
+  const AttnArgs& a = t.a;
+  constexpr int kWk = kTileWaves / WR;      // key groups
+  constexpr int kSteps = D / 16;            // MFMA k-steps of a score tile
+  constexpr int kDt = D / 32;               // 32-wide head-dim tiles of the output
+  constexpr int kRowLanes = D / 8;          // 16-byte pieces of a row
+  constexpr int kLoads = kRowLanes / WR;    // pieces of a 64-row tile per thread
+  using L = TileLds<D>;
+  __shared__ __attribute__((aligned(16))) char lds[tiled_lds_bytes<D, WR>()];
   const int lane = threadIdx.x & (SF_WAVE - 1);
-  const int wave = threadIdx.x / SF_WAVE;
-  const int g4 = lane >> 4;           // row group of the C layout / k group of A, B
-  const int col = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SF_WAVE);
+  const int kg = wave / WR;
+  const int hf = lane >> 5;
+  const int col = lane & 31;
+  // Consecutive workgroups take different KV heads (an XCD then keeps one or
+  // few heads' K/V in its L2); the last row tiles, which see the most keys
+  // under the causal rule, go first.
   const int h = blockIdx.x % a.Hkv;
-  const int t0 = (blockIdx.x / a.Hkv) * kTok;
-  char* vtile = lds + wave * kKeysPerChunk * kVRow;                       // [32][D] bf16
-  char* ptile = lds + kMfmaWaves * kKeysPerChunk * kVRow + wave * 16 * kPRow;  // [16][32] bf16
+  const int rest = blockIdx.x / a.Hkv;
+  const int split = rest % t.splits;
+  const int block_row = (t.row_tiles - 1 - rest / t.splits) * 32 * WR;
+  const int wave_row = block_row + 32 * (wave % WR);
+  const bool active = wave_row < t.rows;
+  const int row = wave_row + col;
+  const int row_c = min(row, t.rows - 1);
+  const int tok = row_c >> t.log_g;
+  const int head = (h << t.log_g) + (row_c & ((1 << t.log_g) - 1));
 
-  // A operand: query row `col` of the tile (token t0 + col / G, head h G + col % G).
-  uint4 qa[kSteps];
+  // B operand of the scores: this lane's query row.  A negative scale flips
+  // the signs here (exact), so the row maximum is that of the scaled scores.
+  sf_bf16x8 qf[kSteps];
   {
-    const int t = min(t0 + col / G, a.Q - 1);
-    const uint16_t* qr = a.q + t * a.q_tok + static_cast<int64_t>(h * G + col % G) * a.q_head;
+    const uint16_t* qr = a.q + tok * a.q_tok + head * a.q_head + 8 * hf;
+    const uint32_t flip = a.scale < 0.f ? 0x80008000u : 0u;
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s)
-      qa[s] = *reinterpret_cast<const uint4*>(qr + 32 * s + 8 * g4);
+    for (int s = 0; s < kSteps; ++s) qf[s] = __builtin_bit_cast(sf_bf16x8, ld16(qr + 16 * s) ^ flip);
   }
-  // Rows of this lane in the C layout: 4 g4 + i, token t0 + (4 g4 + i) / G.
-  int tok[4];
-  bool row_ok[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    tok[i] = t0 + (4 * g4 + i) / G;
-    row_ok[i] = tok[i] < a.Q;
+  const float c = fabsf(a.scale) * 1.44269504088896341f;  // log2 units
+
+  // Keys: [begin, end) for the workgroup; the wavefront's rows see none from
+  // wave_end on, and all of them see the keys below wave_full.
+  const int last_row = min(block_row + 32 * WR, t.rows) - 1;
+  const int diag = a.S - a.Q + 1;
+  const int begin = split * t.split_keys;
+  int end = min(a.S, begin + t.split_keys);
+  int wave_end = end, wave_full = 0;
+  if (!MASK) {
+    end = min(end, diag + (last_row >> t.log_g));
+    wave_end = min(end, diag + (min(wave_row + 31, t.rows - 1) >> t.log_g));
+    wave_full = diag + (min(wave_row, t.rows - 1) >> t.log_g);
   }
+  const int lane_end = MASK ? a.S : diag + tok;  // keys this lane's row sees (no mask)
   const uint16_t* kh = a.k + h * a.k_head;
   const uint16_t* vh = a.v + h * a.v_head;
-  float m[4], l[4];
-  sf_f32x4 acc[kNt];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.f;
-  }
-#pragma unroll
-  for (int nt = 0; nt < kNt; ++nt) acc[nt] = sf_f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint8_t* mrow = MASK ? a.mask + tok * a.mask_q : nullptr;
 
-  // Chunk loads (keys, value rows, mask bits) are issued one chunk ahead.
-  constexpr int kLanesPerRow = D / 8;
-  constexpr int kRowsPerLoad = SF_WAVE / kLanesPerRow;
-  constexpr int kVLoads = kKeysPerChunk / kRowsPerLoad;
-  constexpr int kStride = kMfmaWaves * kKeysPerChunk;
-  uint4 kf[2][kSteps], vv[kVLoads];
-  uint32_t okbits = 0;  // bit 4 ct + i: key kb + 16 ct + col admitted for row 4 g4 + i
-  auto load_chunk = [&](int kb) {
+  float m = -INFINITY, l = 0.f;  // row maximum (unscaled), this half's sum
+  sf_f32x16 acc[kDt];
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      // Key fragments (B): key kb + 16 ct + col, head-dim 32 s + 8 g4.
-      const uint16_t* kr = kh + min(kb + 16 * ct + col, a.S - 1) * a.k_tok + 8 * g4;
+  for (int dt = 0; dt < kDt; ++dt)
 #pragma unroll
-      for (int s = 0; s < kSteps; ++s) kf[ct][s] = *reinterpret_cast<const uint4*>(kr + 32 * s);
-    }
-    // Value rows kb .. kb + 31 (rows past the end repeat the last key: finite
-    // values that meet p = 0).
+    for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
+
+  // Piece gt + j * 64 WR of a tile: row piece / kRowLanes.
+  const int gt = threadIdx.x % (SF_WAVE * WR);
+  const int ld_row = gt / kRowLanes;
+  const int ld_col = gt % kRowLanes;
+  constexpr int kRowsPerLoad = SF_WAVE * WR / kRowLanes;
+  sf_u32x4 kr[kLoads], vr[kLoads];
+  uint32_t mw[8];
+  const uint32_t k_off = 2 * (ld_row * static_cast<uint32_t>(a.k_tok) + 8 * ld_col);
+  const uint32_t v_off = 2 * (ld_row * static_cast<uint32_t>(a.v_tok) + 8 * ld_col);
+  auto load_tile = [&](int kb) {
+    if (kb + kTileKeys <= a.S) {
+      const uint16_t* kp = kh + kb * a.k_tok;
+      const uint16_t* vp = vh + kb * a.v_tok;
 #pragma unroll
-    for (int j = 0; j < kVLoads; ++j) {
-      const int r = j * kRowsPerLoad + lane / kLanesPerRow;
-      vv[j] = *reinterpret_cast<const uint4*>(vh + min(kb + r, a.S - 1) * a.v_tok +
-                                              8 * (lane % kLanesPerRow));
-    }
-    okbits = 0;
+      for (int j = 0; j < kLoads; ++j) kr[j] = ld16(kp + j * kRowsPerLoad * a.k_tok, k_off);
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      const int key = kb + 16 * ct + col;
+      for (int j = 0; j < kLoads; ++j) vr[j] = ld16(vp + j * kRowsPerLoad * a.v_tok, v_off);
+    } else {
+      // Rows past the end repeat the last key: finite values that meet p = 0.
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        // Rows of one token share its mask byte (consecutive rows 4 g4 + i).
-        bool ok = row_ok[i] && key < a.S;
-        if (ok) ok = a.mask ? a.mask[tok[i] * a.mask_q + key] != 0 : key <= a.S - a.Q + tok[i];
-        okbits |= static_cast<uint32_t>(ok) << (4 * ct + i);
+      for (int j = 0; j < kLoads; ++j) {
+        const int64_t key = min(kb + j * kRowsPerLoad + ld_row, a.S - 1);
+        kr[j] = ld16(kh + key * a.k_tok + 8 * ld_col);
+        vr[j] = ld16(vh + key * a.v_tok + 8 * ld_col);
       }
+    }
+    if (MASK) {
+#pragma unroll
+      for (int g = 0; g < 8; ++g) mw[g] = mask_word(mrow, kb + 8 * g + 4 * hf, a.S);
     }
   };
-  if (wave * kKeysPerChunk < a.S) load_chunk(wave * kKeysPerChunk);
-  for (int kb = wave * kKeysPerChunk; kb < a.S; kb += kStride) {
-    uint4 kc[2][kSteps];
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-      for (int s = 0; s < kSteps; ++s) kc[ct][s] = kf[ct][s];
-    const uint32_t okc = okbits;
-    // The chunk's value rows into this wavefront's LDS tile.
-#pragma unroll
-    for (int j = 0; j < kVLoads; ++j) {
-      const int r = j * kRowsPerLoad + lane / kLanesPerRow;
-      uint2* dst = reinterpret_cast<uint2*>(vtile + r * kVRow + 16 * (lane % kLanesPerRow));
-      dst[0] = make_uint2(vv[j].x, vv[j].y);
-      dst[1] = make_uint2(vv[j].z, vv[j].w);
-    }
-    if (kb + kStride < a.S) load_chunk(kb + kStride);
-    // Scores of the 16 x 32 tile.
-    sf_f32x4 sc[2];
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      sc[ct] = sf_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < kSteps; ++s) sc[ct] = mfma_bf16(qa[s], kc[ct][s], sc[ct]);
-    }
-    // Online softmax per row.
-    float p[2][4];
-    float alpha[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      bool ok[2];
-      float x[2];
-#pragma unroll
-      for (int ct = 0; ct < 2; ++ct) {
-        ok[ct] = (okc >> (4 * ct + i)) & 1u;
-        x[ct] = sc[ct][i] * a.scale;
-      }
-      const float cmax = row16_max(fmaxf(ok[0] ? x[0] : -INFINITY, ok[1] ? x[1] : -INFINITY));
-      const float mnew = fmaxf(m[i], cmax);
-      alpha[i] = 1.f;
-      p[0][i] = p[1][i] = 0.f;
-      if (mnew != -INFINITY) {
-        alpha[i] = m[i] == -INFINITY ? 0.f : __expf(m[i] - mnew);
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct)
-          if (ok[ct]) p[ct][i] = __expf(x[ct] - mnew);
-      }
-      l[i] = l[i] * alpha[i] + row16_sum(p[0][i] + p[1][i]);
-      m[i] = mnew;
-    }
-#pragma unroll
-    for (int nt = 0; nt < kNt; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[nt][i] *= alpha[i];
-    // P (bf16) through LDS into the A layout: row col, keys 8 g4 .. 8 g4 + 7.
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<uint16_t*>(ptile + (4 * g4 + i) * kPRow + 2 * (16 * ct + col)) =
-            sf_f32_to_bf16(p[ct][i]);
-    // The V and P tiles are this wavefront's own: its LDS accesses run in
-    // order, and the fence keeps the compiler from moving the reads above.
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const uint4 pa = *reinterpret_cast<const uint4*>(ptile + col * kPRow + 16 * g4);
-    // P.V: B = value rows 8 g4 .. 8 g4 + 7 of head-dim column 16 nt + col.
-#pragma unroll
-    for (int nt = 0; nt < kNt; ++nt) {
-      uint32_t w[4];
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const char* v0 = vtile + (8 * g4 + 2 * jj) * kVRow + 2 * (16 * nt + col);
-        const uint32_t lo = *reinterpret_cast<const uint16_t*>(v0);
-        const uint32_t hi = *reinterpret_cast<const uint16_t*>(v0 + kVRow);
-        w[jj] = lo | (hi << 16);
-      }
-      acc[nt] = mfma_bf16(pa, make_uint4(w[0], w[1], w[2], w[3]), acc[nt]);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // tiles reused by the next chunk
-  }
 
-  // Merge the wavefront states in wavefront order.  The merge state overlays
-  // the tiles of every wavefront: all of them have left the chunk loop first.
-  __syncthreads();
-  float* mst = reinterpret_cast<float*>(lds);                        // [waves][16] max
-  float* lst = mst + kMfmaWaves * 16;                                 // [waves][16] sum
-  float* ast = lst + kMfmaWaves * 16;                                 // [waves][16][D] acc
-  if (col == 0) {
+  int kb = begin + kg * kTileKeys;
+  if (kb < end) load_tile(kb);
+  char* tile = lds + kg * L::bytes;
+  int buf = 0;
+  for (; kb < end; kb += kTileKeys * kWk) {
+    if (WR == 4) tile = lds + (buf ^= 1) * L::bytes;
+    char* ktile = tile;
+    char* vtile = tile + kTileKeys * L::krow;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      mst[wave * 16 + 4 * g4 + i] = m[i];
-      lst[wave * 16 + 4 * g4 + i] = l[i];
+    for (int j = 0; j < kLoads; ++j) {
+      const int r = j * kRowsPerLoad + ld_row;
+      *reinterpret_cast<sf_u32x4*>(ktile + r * L::krow + 16 * ld_col) = kr[j];
+      *reinterpret_cast<sf_u32x4*>(vtile + r * L::vrow + 16 * ld_col) = vr[j];
     }
-  }
+    uint32_t mc[8];
+    if (MASK) {
 #pragma unroll
-  for (int nt = 0; nt < kNt; ++nt)
+      for (int g = 0; g < 8; ++g) mc[g] = mw[g];
+    }
+    if (kb + kTileKeys * kWk < end) load_tile(kb + kTileKeys * kWk);
+    if (WR == 4)
+      __syncthreads();  // the tile is complete; the other buffer's reads are done
+    else
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (active && kb < wave_end) {
+      sf_f32x16 s[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ast[(wave * 16 + 4 * g4 + i) * D + 16 * nt + col] = acc[nt][i];
-  __syncthreads();
-  const int Hq = a.Hkv * G;
-  for (int o = threadIdx.x; o < 16 * D; o += kMfmaWaves * SF_WAVE) {
-    const int r = o / D;
-    const int d = o - r * D;
-    const int t = t0 + r / G;
-    if (t >= a.Q) continue;
-    float M = -INFINITY;
+      for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
-    for (int w = 0; w < kMfmaWaves; ++w) M = fmaxf(M, mst[w * 16 + r]);
-    float L = 0.f, O = 0.f;
-    if (M != -INFINITY) {
+        for (int i = 0; i < 16; ++i) s[kt][i] = 0.f;
 #pragma unroll
-      for (int w = 0; w < kMfmaWaves; ++w) {
-        const float mw = mst[w * 16 + r];
-        if (mw == -INFINITY) continue;
-        const float f = __expf(mw - M);
-        L = __builtin_fmaf(lst[w * 16 + r], f, L);
-        O = __builtin_fmaf(ast[(w * 16 + r) * D + d], f, O);
+        for (int st = 0; st < kSteps; ++st) {
+          const sf_bf16x8 kf = *reinterpret_cast<const sf_bf16x8*>(
+              ktile + (32 * kt + col) * L::krow + 32 * st + 16 * hf);
+          s[kt] = mfma_32(kf, qf[st], s[kt]);
+        }
+      }
+      // Keys the row does not admit: -inf (their p is 0).
+      if (MASK) {
+        bool all = true;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) all = all && mc[g] == 0x01010101u;
+        if (!__all(all)) {
+#pragma unroll
+          for (int g = 0; g < 8; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (!((mc[g] >> (8 * i)) & 0xffu)) s[g >> 2][4 * (g & 3) + i] = -INFINITY;
+        }
+      } else if (kb + kTileKeys > wave_full) {
+#pragma unroll
+        for (int g = 0; g < 8; ++g)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (kb + 8 * g + 4 * hf + i >= lane_end) s[g >> 2][4 * (g & 3) + i] = -INFINITY;
+      }
+      float mx[2] = {s[0][0], s[1][0]};
+#pragma unroll
+      for (int i = 1; i < 16; ++i)
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) mx[kt] = max_raw(mx[kt], s[kt][i]);
+      const float mnew = fmaxf(m, half_max(max_raw(mx[0], mx[1])));
+      if (__any(mnew > m)) {
+        const float alpha =
+            m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m * c - mnew * c);
+        l *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
+        m = mnew;
+      }
+      const float base = m == -INFINITY ? 0.f : -(m * c);
+      uint32_t pk[2][8];
+      float sum[2] = {0.f, 0.f};
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][i], c, base));
+          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][i + 1], c, base));
+          sum[0] += p0;
+          sum[1] += p1;
+          pk[kt][i >> 1] = pack_bf16(p0, p1);
+        }
+      l += sum[0] + sum[1];
+      const char* vlane = vtile + (4 * hf + ((lane & 15) >> 2)) * L::vrow +
+                          32 * ((lane >> 4) & 1) + 8 * (lane & 3);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const sf_u32x4 pw = {pk[ks >> 1][4 * (ks & 1)], pk[ks >> 1][4 * (ks & 1) + 1],
+                             pk[ks >> 1][4 * (ks & 1) + 2], pk[ks >> 1][4 * (ks & 1) + 3]};
+        const sf_bf16x8 pf = __builtin_bit_cast(sf_bf16x8, pw);
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt) {
+          struct { sf_i16x4 lo, hi; } vf;
+          vf.lo = read_tr4(vlane + 16 * ks * L::vrow + 64 * dt);
+          vf.hi = read_tr4(vlane + (16 * ks + 8) * L::vrow + 64 * dt);
+          acc[dt] = mfma_32(__builtin_bit_cast(sf_bf16x8, vf), pf, acc[dt]);
+        }
       }
     }
-    const float out = L > 0.f ? O / L : 0.f;
-    a.out[(static_cast<int64_t>(t) * Hq + h * G + r % G) * D + d] = sf_f32_to_bf16(out);
+    if (WR != 4) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // tile reused
+  }
+  l = half_sum(l);
+  const float mlog = m == -INFINITY ? -INFINITY : m * c;
+
+  const int64_t part_row = (static_cast<int64_t>(split) * a.Hkv + h) * t.rows;
+  if (WR == 4) {
+    if (row >= t.rows) return;
+    if (t.splits > 1) {
+      if (hf == 0) t.part_ml[part_row + row] = make_float2(mlog, l);
+      if (mlog == -INFINITY) return;  // never read
+      float* o = t.part_acc + (part_row + row) * D + 4 * hf;
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<float4*>(o + 32 * dt + 8 * g) =
+              make_float4(acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]);
+      return;
+    }
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float o[4] = {acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
+        store_row4(t, h, row, D, 32 * dt + 8 * g + 4 * hf, o, l);
+      }
+  } else {
+    // Merge the key groups in order.  Their state overlays every tile.
+    __syncthreads();
+    constexpr int kRows = 32 * WR;
+    float* sacc = reinterpret_cast<float*>(lds);                 // [kWk][kRows][orow]
+    float* sml = sacc + kWk * kRows * L::orow;                   // [kWk][kRows][2]
+    const int lrow = kg * kRows + 32 * (wave % WR) + col;
+    if (hf == 0) {
+      sml[2 * lrow] = mlog;
+      sml[2 * lrow + 1] = l;
+    }
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4*>(sacc + lrow * L::orow + 32 * dt + 8 * g + 4 * hf) =
+            make_float4(acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kRows * (D / 4); i += kTileThreads) {
+      const int lr = i / (D / 4);
+      const int d = 4 * (i % (D / 4));
+      const int r = block_row + lr;
+      if (r >= t.rows) break;
+      float M = -INFINITY, sum = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kWk; ++w) M = fmaxf(M, sml[2 * (w * kRows + lr)]);
+#pragma unroll
+      for (int w = 0; w < kWk; ++w) {
+        const float wm = sml[2 * (w * kRows + lr)];
+        if (wm == -INFINITY) continue;
+        add_state(wm, sml[2 * (w * kRows + lr) + 1],
+                  *reinterpret_cast<const float4*>(sacc + (w * kRows + lr) * L::orow + d), M, sum, o);
+      }
+      if (t.splits > 1) {
+        if (d == 0) t.part_ml[part_row + r] = make_float2(M, sum);
+        *reinterpret_cast<float4*>(t.part_acc + (part_row + r) * D + d) =
+            make_float4(o[0], o[1], o[2], o[3]);
+      } else {
+        store_row4(t, h, r, D, d, o, sum);
+      }
+    }
   }
 }
 
-template <int G, int D>
-int launch_mfma(const AttnArgs& a, hipStream_t s) {
-  constexpr int kTok = 16 / G;
-  const dim3 grid(static_cast<unsigned>((a.Q + kTok - 1) / kTok) * a.Hkv);
-  tree_attention_mfma_kernel<G, D><<<grid, dim3(kMfmaWaves * SF_WAVE), 0, s>>>(a);
+// Merges the key splits of every query row in split order.  A row's D / 4
+// threads read its splits' accumulators with all loads in flight at once: one
+// group of threads for up to 8 splits, eight groups (merged through LDS, in
+// group order) above.
+constexpr int kMergeDepth = 8;  // splits per group
+
+template <int D, int GROUPS>
+__global__ __launch_bounds__(kTileThreads) void tree_attention_merge_kernel(const TiledArgs t) {
+  constexpr int kLanes = D / 4;
+  constexpr int kSubs = kTileThreads / kLanes;
+  constexpr int kRows = kSubs / GROUPS;
+  static_assert(GROUPS * kMergeDepth <= kMaxSplits, "splits per row");
+  __shared__ float sml[kSubs][2];
+  __shared__ float4 sacc[GROUPS > 1 ? kSubs : 1][kLanes];
+  const AttnArgs& a = t.a;
+  const int sub = threadIdx.x / kLanes;
+  const int dl = threadIdx.x % kLanes;
+  const int g = sub % GROUPS;
+  const int64_t total = static_cast<int64_t>(a.Hkv) * t.rows;
+  const int64_t hr = static_cast<int64_t>(blockIdx.x) * kRows + sub / GROUPS;
+  const bool valid = hr < total;
+  const int64_t base = valid ? hr : 0;
+  float2 ml[kMergeDepth];
+  float4 v[kMergeDepth];
+#pragma unroll
+  for (int j = 0; j < kMergeDepth; ++j) {
+    const int s = g + GROUPS * j;
+    ml[j] = make_float2(-INFINITY, 0.f);
+    v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (s < t.splits) {
+      ml[j] = t.part_ml[s * total + base];
+      // Not written (and not used) where the split admits no key of the row.
+      v[j] = *reinterpret_cast<const float4*>(t.part_acc + (s * total + base) * D + 4 * dl);
+    }
+  }
+  float M = -INFINITY, sum = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < kMergeDepth; ++j) M = fmaxf(M, ml[j].x);
+#pragma unroll
+  for (int j = 0; j < kMergeDepth; ++j) {
+    if (ml[j].x == -INFINITY) continue;
+    add_state(ml[j].x, ml[j].y, v[j], M, sum, o);
+  }
+  if (GROUPS > 1) {
+    if (dl == 0) {
+      sml[sub][0] = M;
+      sml[sub][1] = sum;
+    }
+    sacc[sub][dl] = make_float4(o[0], o[1], o[2], o[3]);
+    __syncthreads();
+    if (g != 0) return;
+    M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < GROUPS; ++w) M = fmaxf(M, sml[sub + w][0]);
+    sum = o[0] = o[1] = o[2] = o[3] = 0.f;
+#pragma unroll
+    for (int w = 0; w < GROUPS; ++w) {
+      if (sml[sub + w][0] == -INFINITY) continue;
+      add_state(sml[sub + w][0], sml[sub + w][1], sacc[sub + w][dl], M, sum, o);
+    }
+  }
+  if (valid) store_row4(t, static_cast<int>(hr / t.rows), static_cast<int>(hr % t.rows), D, 4 * dl, o, sum);
+}
+
+bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
+
+// c = |scale| log2(e) must be a normal finite number: a masked score of -inf
+// times 0 would be NaN.
+bool scale_ok(float scale) {
+  const float c = __builtin_fabsf(scale) * 1.44269504088896341f;
+  return c >= 1.17549435e-38f && c <= 3.0e38f;
+}
+
+// Row groups (WR) and key splits of a call.
+struct TiledPlan {
+  int wr, row_tiles, splits, split_keys;
+};
+
+// The form and split with the least estimated time.  A workgroup's step (one
+// 64-key tile at WR = 4, four at WR = 1) takes about 1.2 / 2.4 us on MI355X,
+// 1.6 / 2.9 us with a mask; splitting adds the merge launch (2.5 us) and the
+// partial states' way through memory (0.28 ns per row and split, 1 KiB each);
+// a CU runs one WR = 1 workgroup at a time, and WR = 4 workgroups above 1.5
+// per CU wait for each other.  Measured at 32 query / 4 KV heads of 128 (us):
+//   1 query, 4096 keys:     82.6 unsplit, 9.3 in 33 splits (WR = 4)
+//   32 queries, 1056 keys:  21.8 unsplit, 12.2 in 5 (WR = 1); 13.4 WR = 4
+//   61 queries, 1085 keys:  22.0 unsplit, 15.9 in 3, 20.2 in 5 (WR = 1)
+//   129 queries, 8129 keys: 227 unsplit, 46.8 in 11, 54.3 in 32 (WR = 4)
+//   256 queries and keys:   8.8 unsplit (WR = 1), 10.9 (WR = 4), 13.9 in 2
+TiledPlan tiled_plan(int queries, int keys, int kv_heads, int G, bool mask) {
+  const int64_t rows = static_cast<int64_t>(queries) * G;
+  TiledPlan best{};
+  double best_cost = 0.0;
+  for (int wr = 4; wr >= 1; wr -= 3) {
+    const int unit = kTileKeys * (kTileWaves / wr);
+    const int units = (keys + unit - 1) / unit;
+    const int64_t row_tiles = (rows + 32 * wr - 1) / (32 * wr);
+    const int64_t blocks = row_tiles * kv_heads;
+    const double step = wr == 4 ? (mask ? 1.6 : 1.2) : (mask ? 2.9 : 2.4);
+    const int most = units < kMaxSplits ? units : kMaxSplits;
+    int last = 0;
+    for (int want = 1; want <= most; ++want) {
+      const int per = (units + want - 1) / want;
+      const int splits = (units + per - 1) / per;
+      if (splits == last) continue;
+      last = splits;
+      const double total = static_cast<double>(blocks) * splits;
+      double turns = wr == 4 ? total / 384.0 : __builtin_ceil(total / 256.0);
+      if (turns < 1.0) turns = 1.0;
+      double cost = per * step * turns + (wr == 4 ? 0.0 : 0.4);
+      if (splits > 1) cost += 2.5 + 0.28e-3 * static_cast<double>(rows) * kv_heads * splits;
+      if (best.wr && cost >= best_cost) continue;
+      best_cost = cost;
+      best = TiledPlan{wr, static_cast<int>(row_tiles), splits, per * unit};
+      if (total > 2048) break;  // the chip is full: more splits only add to the merge
+    }
+  }
+  return best;
+}
+
+int64_t tiled_workspace(const TiledPlan& p, int queries, int q_heads, int head_dim) {
+  if (p.splits == 1) return 0;
+  return static_cast<int64_t>(p.splits) * queries * q_heads * (head_dim + 2) * 4;
+}
+
+template <int D>
+int launch_tiled(const AttnArgs& a, int G, void* workspace, int64_t workspace_bytes, hipStream_t s) {
+  TiledPlan p = tiled_plan(a.Q, a.S, a.Hkv, G, a.mask != nullptr);
+  const int64_t need = tiled_workspace(p, a.Q, a.Hkv * G, D);
+  if (need > workspace_bytes || (need && (!workspace || !aligned(workspace, 16)))) {
+    p.splits = 1;
+    p.split_keys = a.S;
+  }
+  TiledArgs t{};
+  t.a = a;
+  t.log_g = __builtin_ctz(G);
+  t.rows = a.Q * G;
+  t.row_tiles = p.row_tiles;
+  t.splits = p.splits;
+  t.split_keys = p.split_keys;
+  if (p.splits > 1) {
+    t.part_acc = static_cast<float*>(workspace);
+    t.part_ml = reinterpret_cast<float2*>(
+        t.part_acc + static_cast<int64_t>(p.splits) * a.Hkv * t.rows * D);
+  }
+  const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(p.row_tiles) * a.Hkv * p.splits));
+  const dim3 block(kTileThreads);
+  if (p.wr == 4) {
+    if (a.mask) tree_attention_tiled_kernel<D, 4, true><<<grid, block, 0, s>>>(t);
+    else tree_attention_tiled_kernel<D, 4, false><<<grid, block, 0, s>>>(t);
+  } else {
+    if (a.mask) tree_attention_tiled_kernel<D, 1, true><<<grid, block, 0, s>>>(t);
+    else tree_attention_tiled_kernel<D, 1, false><<<grid, block, 0, s>>>(t);
+  }
   SF_LAUNCH_CHECK();
+  if (p.splits > 1) {
+    constexpr int kSubs = kTileThreads / (D / 4);
+    const int64_t total = static_cast<int64_t>(a.Hkv) * t.rows;
+    if (p.splits <= kMergeDepth)
+      tree_attention_merge_kernel<D, 1><<<dim3(static_cast<unsigned>((total + kSubs - 1) / kSubs)), block, 0, s>>>(t);
+    else
+      tree_attention_merge_kernel<D, 8><<<dim3(static_cast<unsigned>((total + kSubs / 8 - 1) / (kSubs / 8))), block, 0, s>>>(t);
+    SF_LAUNCH_CHECK();
+  }
   return SF_OK;
 }
 
@@ -574,16 +891,16 @@ int launch_g(const AttnArgs& a, hipStream_t s) {
   return SF_OK;
 }
 
-bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
-
 }  // namespace
 
-extern "C" int sf_tree_attention(const void* q, int64_t q_stride_token, int64_t q_stride_head,
-                                 const void* k, int64_t k_stride_head, int64_t k_stride_token,
-                                 const void* v, int64_t v_stride_head, int64_t v_stride_token,
-                                 const uint8_t* mask, int64_t mask_stride_query, int queries,
-                                 int keys, int q_heads, int kv_heads, int head_dim, float scale,
-                                 void* out, sf_stream_t stream) {
+namespace {
+
+int attention_call(const void* q, int64_t q_stride_token, int64_t q_stride_head, const void* k,
+                   int64_t k_stride_head, int64_t k_stride_token, const void* v,
+                   int64_t v_stride_head, int64_t v_stride_token, const uint8_t* mask,
+                   int64_t mask_stride_query, int queries, int keys, int q_heads, int kv_heads,
+                   int head_dim, float scale, void* out, void* workspace, int64_t workspace_bytes,
+                   hipStream_t s) {
   if (queries < 1 || keys < 1 || q_heads < 1 || kv_heads < 1 || head_dim < 1)
     return SF_ERR_INVALID_ARGUMENT;
   if (!q || !k || !v || !out) return SF_ERR_INVALID_ARGUMENT;
@@ -620,29 +937,16 @@ extern "C" int sf_tree_attention(const void* q, int64_t q_stride_token, int64_t 
   a.D = head_dim;
   a.scale = scale;
   a.out = static_cast<uint16_t*>(out);
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // The MFMA form: 16-byte aligned query / key / value rows (8-element
-  // strides), head dim 64 or 128, 2..16 query heads per KV head.
-  const bool rows16 = aligned(q, 16) && aligned(k, 16) && aligned(v, 16) &&
-                      q_stride_token % 8 == 0 && q_stride_head % 8 == 0 &&
-                      v_stride_token % 8 == 0 && v_stride_head % 8 == 0;
-  if (rows16 && head_dim == 128) {
-    switch (G) {
-      case 2: return launch_mfma<2, 128>(a, s);
-      case 4: return launch_mfma<4, 128>(a, s);
-      case 8: return launch_mfma<8, 128>(a, s);
-      case 16: return launch_mfma<16, 128>(a, s);
-      default: break;
-    }
-  } else if (rows16 && head_dim == 64) {
-    switch (G) {
-      case 2: return launch_mfma<2, 64>(a, s);
-      case 4: return launch_mfma<4, 64>(a, s);
-      case 8: return launch_mfma<8, 64>(a, s);
-      case 16: return launch_mfma<16, 64>(a, s);
-      default: break;
-    }
-  }
+  // The tiled form: 16-byte aligned query / key / value rows (8-element
+  // strides), head dim 64 or 128, 2..16 query heads per KV head, and a scale
+  // its log2 units can hold.
+  const bool tiled = aligned(q, 16) && aligned(v, 16) && aligned(out, 8) &&
+                     q_stride_token % 8 == 0 && q_stride_head % 8 == 0 &&
+                     v_stride_token % 8 == 0 && v_stride_head % 8 == 0 && k_stride_token < (1 << 24) &&
+                     v_stride_token < (1 << 24) && G >= 2 && G <= 16 && (G & (G - 1)) == 0 && scale_ok(scale) &&
+                     static_cast<int64_t>(queries) * G <= 0x3fffffff;
+  if (tiled && head_dim == 128) return launch_tiled<128>(a, G, workspace, workspace_bytes, s);
+  if (tiled && head_dim == 64) return launch_tiled<64>(a, G, workspace, workspace_bytes, s);
   switch (G) {
     case 1: return launch_g<1>(a, s);
     case 2: return launch_g<2>(a, s);
@@ -651,4 +955,43 @@ extern "C" int sf_tree_attention(const void* q, int64_t q_stride_token, int64_t 
     case 16: return launch_g<16>(a, s);
     default: return SF_ERR_UNSUPPORTED_SHAPE;
   }
+}
+
+}  // namespace
+
+extern "C" int sf_tree_attention(const void* q, int64_t q_stride_token, int64_t q_stride_head,
+                                 const void* k, int64_t k_stride_head, int64_t k_stride_token,
+                                 const void* v, int64_t v_stride_head, int64_t v_stride_token,
+                                 const uint8_t* mask, int64_t mask_stride_query, int queries,
+                                 int keys, int q_heads, int kv_heads, int head_dim, float scale,
+                                 void* out, sf_stream_t stream) {
+  return attention_call(q, q_stride_token, q_stride_head, k, k_stride_head, k_stride_token, v,
+                        v_stride_head, v_stride_token, mask, mask_stride_query, queries, keys,
+                        q_heads, kv_heads, head_dim, scale, out, nullptr, 0,
+                        reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int64_t sf_tree_attention_workspace(int queries, int keys, int q_heads, int kv_heads,
+                                               int head_dim, int masked) {
+  if (queries < 1 || keys < 1 || kv_heads < 1 || q_heads < kv_heads || q_heads % kv_heads) return 0;
+  const int G = q_heads / kv_heads;
+  if ((head_dim != 64 && head_dim != 128) || G > 16 ||
+      static_cast<int64_t>(queries) * G > 0x3fffffff)
+    return 0;
+  return tiled_workspace(tiled_plan(queries, keys, kv_heads, G, masked != 0), queries, q_heads, head_dim);
+}
+
+extern "C" int sf_tree_attention_split(const void* q, int64_t q_stride_token,
+                                       int64_t q_stride_head, const void* k,
+                                       int64_t k_stride_head, int64_t k_stride_token,
+                                       const void* v, int64_t v_stride_head,
+                                       int64_t v_stride_token, const uint8_t* mask,
+                                       int64_t mask_stride_query, int queries, int keys,
+                                       int q_heads, int kv_heads, int head_dim, float scale,
+                                       void* out, void* workspace, int64_t workspace_bytes,
+                                       sf_stream_t stream) {
+  return attention_call(q, q_stride_token, q_stride_head, k, k_stride_head, k_stride_token, v,
+                        v_stride_head, v_stride_token, mask, mask_stride_query, queries, keys,
+                        q_heads, kv_heads, head_dim, scale, out, workspace, workspace_bytes,
+                        reinterpret_cast<hipStream_t>(stream));
 }

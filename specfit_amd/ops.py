@@ -8,6 +8,7 @@ C-ABI.  There is no PyTorch or CPU fallback.
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 from typing import Sequence
 
@@ -251,7 +252,7 @@ def _stream_handle(stream: torch.cuda.Stream | None, device: torch.device) -> in
 def _require_cuda(name: str, t: torch.Tensor, dtype: torch.dtype | None = None) -> None:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be on a HIP device")
     if dtype is not None and t.dtype != dtype:
         raise ValueError(f"{name} must have dtype {dtype}")
@@ -678,6 +679,15 @@ def expert_decode(record: torch.Tensor, counts, table: bytes, out: torch.Tensor,
 
 
 # ------------------------------------------------------------------ K5 ----
+@functools.lru_cache(maxsize=256)
+def _attention_workspace(queries: int, keys: int, q_heads: int, kv_heads: int, head_dim: int,
+                         masked: bool) -> int:
+    """Scratch bytes of a K5 call, a function of its sizes alone (the layers
+    of one forward ask for the same one)."""
+    return _native.lib().sf_tree_attention_workspace(queries, keys, q_heads, kv_heads, head_dim,
+                                                     masked)
+
+
 def tree_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                    mask: torch.Tensor | None, scale: float, *,
                    stream: torch.cuda.Stream | None = None) -> torch.Tensor:
@@ -698,28 +708,45 @@ def tree_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
         raise ValueError("key/value shapes do not match the query")
     if Hkv < 1 or Hq % Hkv:
         raise ValueError("query heads must be a multiple of key/value heads")
+    device = query.device
+    mask_ptr, mask_batch, mask_q = None, 0, 0
     if mask is not None:
         if mask.dtype != torch.bool:
             raise TypeError("tree attention takes a bool mask (True = attend)")
-        if mask.device != query.device or mask.dim() != 4 or mask.shape[0] not in (1, B) \
+        if mask.device != device or mask.dim() != 4 or mask.shape[0] not in (1, B) \
                 or tuple(mask.shape[2:]) != (Q, S) or mask.stride(-1) != 1:
             raise ValueError(f"mask must be bool [B, 1, {Q}, {S}] with a unit last stride")
-    out = torch.empty((B, Q, Hq, D), dtype=_BF16, device=query.device)
+        mask_batch, _, mask_q, _ = mask.stride()
+        if mask.shape[0] != B:
+            mask_batch = 0
+    out = torch.empty((B, Q, Hq, D), dtype=_BF16, device=device)
     if B == 0 or Q == 0:
         return out
     if S == 0:
         return out.zero_()
     lib = _native.lib()
-    handle = _stream_handle(stream, query.device)
+    handle = _stream_handle(stream, device)
+    # Scratch of a call whose keys are split over the chip; the calls of a
+    # batch run one after another on the stream and share it.
+    need = _attention_workspace(Q, S, Hq, Hkv, D, mask is not None)
+    work_ptr = None
+    if need:
+        work = torch.empty(need, dtype=torch.uint8, device=device)
+        work_ptr = work.data_ptr()
+        if stream is not None:  # may not be the stream the memory was allocated on
+            work.record_stream(stream)
+    # Addresses and strides instead of per-batch views: this call is often
+    # shorter on the device than a handful of tensor operations on the host.
+    (qb, qh, qt, _), (kb, kh, kt, _), (vb, vh, vt, _) = query.stride(), key.stride(), value.stride()
+    q_ptr, k_ptr, v_ptr, out_ptr = query.data_ptr(), key.data_ptr(), value.data_ptr(), out.data_ptr()
+    if mask is not None:
+        mask_ptr = mask.data_ptr()
     for b in range(B):
-        q, k, v = query[b], key[b], value[b]
-        m = None if mask is None else mask[b if mask.shape[0] == B else 0, 0]
-        rc = lib.sf_tree_attention(
-            q.data_ptr(), q.stride(1), q.stride(0), k.data_ptr(), k.stride(0), k.stride(1),
-            v.data_ptr(), v.stride(0), v.stride(1), None if m is None else m.data_ptr(),
-            0 if m is None else m.stride(0), Q, S, Hq, Hkv, D, float(scale), out[b].data_ptr(),
-            handle)
-        _native.check(rc, "sf_tree_attention")
+        rc = lib.sf_tree_attention_split(
+            q_ptr + 2 * b * qb, qt, qh, k_ptr + 2 * b * kb, kh, kt, v_ptr + 2 * b * vb, vh, vt,
+            None if mask_ptr is None else mask_ptr + b * mask_batch, mask_q, Q, S, Hq, Hkv, D,
+            float(scale), out_ptr + 2 * b * Q * Hq * D, work_ptr, need, handle)
+        _native.check(rc, "sf_tree_attention_split")
     return out
 
 

@@ -173,8 +173,8 @@ def summarize(fetch_dir: str, write_dir: str, command: str | None = None) -> str
 LIBRARY_KERNELS = ("router_logits_kernel", "router_select_kernel", "dispatch_kernel",
                    "gateup_mfma_kernel", "down_mfma_kernel", "gateup_generic_kernel",
                    "down_generic_kernel", "combine_kernel", "decode_kernel",
-                   "tree_attention_kernel", "tree_attention_mfma_kernel", "rms_norm_kernel",
-                   "qk_norm_rope_kernel", "router_topk_scalar_kernel")
+                   "tree_attention_kernel", "tree_attention_tiled_kernel",
+                   "tree_attention_merge_kernel", "rms_norm_kernel", "qk_norm_rope_kernel", "router_topk_scalar_kernel")
 
 
 FORWARD_START = "router_logits_kernel"

@@ -73,6 +73,15 @@ def test_host_side_validation_needs_no_device():
     assert attn(32, 4, 512) == 2
     assert attn(96, 4, 128) == 2          # 24 query heads per key/value head
     assert attn(32, 4, 128, k=fake + 8) == 3
+    # split scratch: none for shapes that do not split or do not exist, else whole states
+    # of head_dim + 2 floats per row and split
+    work = lib.sf_tree_attention_workspace
+    assert work(4096, 4096, 32, 4, 128, 0) == 0 and work(1, 16, 32, 4, 128, 0) == 0
+    assert work(1, 4096, 32, 5, 128, 0) == 0 and work(0, 4096, 32, 4, 128, 0) == 0
+    assert work(1, 4096, 32, 4, 96, 0) == 0
+    for queries, keys, masked in [(1, 4096, 0), (1, 1 << 30, 0), (61, 1085, 1), (129, 8129, 1)]:
+        splits, rest = divmod(work(queries, keys, 32, 4, 128, masked), queries * 32 * 130 * 4)
+        assert rest == 0 and 2 <= splits <= 64, (queries, keys)
     # query/key norm + rotary: head dim, token strides shorter than the heads or unaligned
     def qk(q_tok, k_tok, head_dim=128, tokens=2):
         return lib.sf_qk_norm_rope(fake, q_tok, fake, k_tok, tokens, 32, 4, head_dim, fake, fake,

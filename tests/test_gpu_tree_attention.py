@@ -112,6 +112,46 @@ def test_mfma_and_loop_kernels_agree(device):
     assert ((fast.float() - loop.float()).abs().max() / ref.abs().max()).item() <= 1e-2
 
 
+# Edges of the tiled form: 64-key tiles and 32- / 128-row tiles with remainders,
+# keys fewer than queries (rows without a key give 0), one to many key splits,
+# both forms with and without a mask, negative scales.
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 4, 128), (8, 4, 64), (16, 1, 64)])
+@pytest.mark.parametrize("Q,S,scale", [(1, 63, 0.09), (1, 65, -0.09), (1, 4097, 0.09), (3, 2, 0.09),
+                                       (17, 129, 0.1), (33, 1500, -0.1), (70, 64, 0.09),
+                                       (129, 3000, 0.09), (300, 300, 0.09)])
+def test_tiled_edges(device, Hq, Hkv, D, Q, S, scale):
+    g = torch.Generator().manual_seed(Q * 7 + S + D)
+    q = _rand((2, Q, Hq, D + 8), device, g)[..., :D].transpose(1, 2)  # padded token rows
+    k = _rand((2, S, Hkv, D), device, g).transpose(1, 2)
+    v = _rand((2, Hkv, S, D + 16), device, g)[..., :D]
+    ref = _reference(q, k, v, None, scale)
+    _check(ops.tree_attention(q, k, v, None, scale), ref)
+    mask = (torch.rand((2, 1, Q, S + 3), generator=g) < 0.4).to(device)[..., 1:S + 1]
+    mask[..., S // 2] = True
+    out = ops.tree_attention(q, k, v, mask, scale)
+    _check(out, _reference(q, k, v, mask, scale))
+    assert torch.equal(out, ops.tree_attention(q, k, v, mask, scale))
+
+
+def test_split_and_unsplit_calls_agree(device):
+    """A call without scratch memory runs its keys in one split: the same
+    values up to the order of the fp32 sums (one bf16 step of the result)."""
+    from specfit_amd import _native
+
+    g = torch.Generator().manual_seed(31)
+    Hq, Hkv, D, Q, S = 32, 4, 128, 2, 3001
+    q, k, v = (_rand(s, device, g) for s in ((Hq, Q, D), (Hkv, S, D), (Hkv, S, D)))
+    assert _native.lib().sf_tree_attention_workspace(Q, S, Hq, Hkv, D, 0) > 0
+    split = ops.tree_attention(q[None], k[None], v[None], None, 0.09)[0]
+    whole = torch.empty((Q, Hq, D), dtype=torch.bfloat16, device=device)
+    rc = _native.lib().sf_tree_attention(
+        q.data_ptr(), D, Q * D, k.data_ptr(), S * D, D, v.data_ptr(), S * D, D, None, 0, Q, S, Hq,
+        Hkv, D, 0.09, whole.data_ptr(), torch.cuda.current_stream(device).cuda_stream)
+    _native.check(rc, "sf_tree_attention")
+    # P is bf16 relative to the running maximum, which differs between the forms.
+    _check(split[None], whole[None].float())
+
+
 def test_fully_masked_row_is_zero_and_large_logits_are_stable(device):
     g = torch.Generator().manual_seed(2)
     q = _rand((1, 8, 5, 128), device, g, std=30.0)
