@@ -127,6 +127,20 @@ def test_dispatch_duplicates_skew_and_invalid(device):
     assert int(plan.fetch_counts()[0][128]) == 2
 
 
+@pytest.mark.parametrize("T,K,E", [(2048, 8, 128),      # 16 spans of one chunk
+                                   (2049, 8, 127),      # a 17th span of 8 routes
+                                   (32768, 8, 256),     # the most spans of one chunk
+                                   (32769, 8, 1),       # spans of two chunks, one id
+                                   (40001, 9, 200)])    # the last span ends inside a chunk
+def test_dispatch_many_spans(device, T, K, E):
+    rng = np.random.default_rng(T)
+    idx = np.minimum(rng.integers(0, 2 * E, size=(T, K)), E - 1).astype(np.int64)  # skewed
+    _dispatch_case(device, idx, E)
+    idx[rng.random((T, K)) < 0.01] = -1  # invalid ids in every span
+    idx[-1, -1] = E
+    _dispatch_case(device, idx, E)
+
+
 def test_dispatch_empty(device):
     plan = ops.dispatch(torch.zeros((0, 8), dtype=torch.int64, device=device), 128)
     assert plan.fetch_counts()[0].sum().item() == 0
