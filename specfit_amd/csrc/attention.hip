@@ -352,7 +352,8 @@ __device__ __forceinline__ sf_u32x4 ld16(const uint16_t* p) {
 }
 
 __device__ __forceinline__ sf_u32x4 ld16(const uint16_t* p, uint32_t byte_offset) {
-  return *(const __attribute__((address_space(1))) sf_u32x4*)(reinterpret_cast<const char*>(p) + byte_offset);
+  return *(const __attribute__((address_space(1))) sf_u32x4*)(reinterpret_cast<const char*>(p) +
+                                                             byte_offset);
 }
 
 // max(x, y) as one instruction: fmaxf first canonicalises operands that come
@@ -370,18 +371,25 @@ __device__ __forceinline__ sf_i16x4 read_tr4(const char* p) {
 
 // Value of the lane 32 away combined with the own one.
 __device__ __forceinline__ float half_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
+  const int v = __float_as_int(x);
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
   return fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
 }
 
 __device__ __forceinline__ float half_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
+  const int v = __float_as_int(x);
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
   return __int_as_float(r[0]) + __int_as_float(r[1]);
 }
 
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   const sf_bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
   return __builtin_bit_cast(uint32_t, v);
+}
+
+// Registers 4 g .. 4 g + 3 of an accumulator: four consecutive head-dim elements.
+__device__ __forceinline__ float4 quad(const sf_f32x16& a, int g) {
+  return make_float4(a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]);
 }
 
 // Mask bytes of keys key .. key + 3 of one row (0 past the last key).
@@ -457,7 +465,8 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
     const uint16_t* qr = a.q + tok * a.q_tok + head * a.q_head + 8 * hf;
     const uint32_t flip = a.scale < 0.f ? 0x80008000u : 0u;
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) qf[s] = __builtin_bit_cast(sf_bf16x8, ld16(qr + 16 * s) ^ flip);
+    for (int s = 0; s < kSteps; ++s)
+      qf[s] = __builtin_bit_cast(sf_bf16x8, ld16(qr + 16 * s) ^ flip);
   }
   const float c = fabsf(a.scale) * 1.44269504088896341f;  // log2 units
 
@@ -635,15 +644,15 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
       for (int dt = 0; dt < kDt; ++dt)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<float4*>(o + 32 * dt + 8 * g) =
-              make_float4(acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]);
+          *reinterpret_cast<float4*>(o + 32 * dt + 8 * g) = quad(acc[dt], g);
       return;
     }
 #pragma unroll
     for (int dt = 0; dt < kDt; ++dt)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const float o[4] = {acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
+        const float4 v = quad(acc[dt], g);
+        const float o[4] = {v.x, v.y, v.z, v.w};
         store_row4(t, h, row, D, 32 * dt + 8 * g + 4 * hf, o, l);
       }
   } else {
@@ -662,7 +671,7 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         *reinterpret_cast<float4*>(sacc + lrow * L::orow + 32 * dt + 8 * g + 4 * hf) =
-            make_float4(acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]);
+            quad(acc[dt], g);
     __syncthreads();
     for (int i = threadIdx.x; i < kRows * (D / 4); i += kTileThreads) {
       const int lr = i / (D / 4);
@@ -677,7 +686,8 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
         const float wm = sml[2 * (w * kRows + lr)];
         if (wm == -INFINITY) continue;
         add_state(wm, sml[2 * (w * kRows + lr) + 1],
-                  *reinterpret_cast<const float4*>(sacc + (w * kRows + lr) * L::orow + d), M, sum, o);
+                  *reinterpret_cast<const float4*>(sacc + (w * kRows + lr) * L::orow + d), M, sum,
+                  o);
       }
       if (t.splits > 1) {
         if (d == 0) t.part_ml[part_row + r] = make_float2(M, sum);
@@ -751,7 +761,8 @@ __global__ __launch_bounds__(kTileThreads) void tree_attention_merge_kernel(cons
       add_state(sml[sub + w][0], sml[sub + w][1], sacc[sub + w][dl], M, sum, o);
     }
   }
-  if (valid) store_row4(t, static_cast<int>(hr / t.rows), static_cast<int>(hr % t.rows), D, 4 * dl, o, sum);
+  if (valid)
+    store_row4(t, static_cast<int>(hr / t.rows), static_cast<int>(hr % t.rows), D, 4 * dl, o, sum);
 }
 
 bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
@@ -770,8 +781,9 @@ struct TiledPlan {
 
 // The form and split with the least estimated time.  A workgroup's step (one
 // 64-key tile at WR = 4, four at WR = 1) takes about 1.2 / 2.4 us on MI355X,
-// 1.6 / 2.9 us with a mask; splitting adds the merge launch (2.5 us) and the
-// partial states' way through memory (0.28 ns per row and split, 1 KiB each);
+// 1.6 / 2.9 us with a mask; splitting adds the merge launch (2.5 us on the
+// device, and 3 us of the caller's time with the scratch allocation, which
+// short calls wait for) and the partial states' way through memory (0.28 ns per row and split, 1 KiB each);
 // a CU runs one WR = 1 workgroup at a time, and WR = 4 workgroups above 1.5
 // per CU wait for each other.  Measured at 32 query / 4 KV heads of 128 (us):
 //   1 query, 4096 keys:     82.6 unsplit, 9.3 in 33 splits (WR = 4)
@@ -800,7 +812,7 @@ TiledPlan tiled_plan(int queries, int keys, int kv_heads, int G, bool mask) {
       double turns = wr == 4 ? total / 384.0 : __builtin_ceil(total / 256.0);
       if (turns < 1.0) turns = 1.0;
       double cost = per * step * turns + (wr == 4 ? 0.0 : 0.4);
-      if (splits > 1) cost += 2.5 + 0.28e-3 * static_cast<double>(rows) * kv_heads * splits;
+      if (splits > 1) cost += 5.5 + 0.28e-3 * static_cast<double>(rows) * kv_heads * splits;
       if (best.wr && cost >= best_cost) continue;
       best_cost = cost;
       best = TiledPlan{wr, static_cast<int>(row_tiles), splits, per * unit};
@@ -816,7 +828,8 @@ int64_t tiled_workspace(const TiledPlan& p, int queries, int q_heads, int head_d
 }
 
 template <int D>
-int launch_tiled(const AttnArgs& a, int G, void* workspace, int64_t workspace_bytes, hipStream_t s) {
+int launch_tiled(const AttnArgs& a, int G, void* workspace, int64_t workspace_bytes,
+                 hipStream_t s) {
   TiledPlan p = tiled_plan(a.Q, a.S, a.Hkv, G, a.mask != nullptr);
   const int64_t need = tiled_workspace(p, a.Q, a.Hkv * G, D);
   if (need > workspace_bytes || (need && (!workspace || !aligned(workspace, 16)))) {
@@ -848,10 +861,10 @@ int launch_tiled(const AttnArgs& a, int G, void* workspace, int64_t workspace_by
   if (p.splits > 1) {
     constexpr int kSubs = kTileThreads / (D / 4);
     const int64_t total = static_cast<int64_t>(a.Hkv) * t.rows;
-    if (p.splits <= kMergeDepth)
-      tree_attention_merge_kernel<D, 1><<<dim3(static_cast<unsigned>((total + kSubs - 1) / kSubs)), block, 0, s>>>(t);
-    else
-      tree_attention_merge_kernel<D, 8><<<dim3(static_cast<unsigned>((total + kSubs / 8 - 1) / (kSubs / 8))), block, 0, s>>>(t);
+    const int64_t rows = p.splits <= kMergeDepth ? kSubs : kSubs / 8;  // of a workgroup
+    const dim3 merge_grid(static_cast<unsigned>((total + rows - 1) / rows));
+    if (p.splits <= kMergeDepth) tree_attention_merge_kernel<D, 1><<<merge_grid, block, 0, s>>>(t);
+    else tree_attention_merge_kernel<D, 8><<<merge_grid, block, 0, s>>>(t);
     SF_LAUNCH_CHECK();
   }
   return SF_OK;
@@ -942,8 +955,9 @@ int attention_call(const void* q, int64_t q_stride_token, int64_t q_stride_head,
   // its log2 units can hold.
   const bool tiled = aligned(q, 16) && aligned(v, 16) && aligned(out, 8) &&
                      q_stride_token % 8 == 0 && q_stride_head % 8 == 0 &&
-                     v_stride_token % 8 == 0 && v_stride_head % 8 == 0 && k_stride_token < (1 << 24) &&
-                     v_stride_token < (1 << 24) && G >= 2 && G <= 16 && (G & (G - 1)) == 0 && scale_ok(scale) &&
+                     v_stride_token % 8 == 0 && v_stride_head % 8 == 0 &&
+                     k_stride_token < (1 << 24) && v_stride_token < (1 << 24) && G >= 2 &&
+                     G <= 16 && (G & (G - 1)) == 0 && scale_ok(scale) &&
                      static_cast<int64_t>(queries) * G <= 0x3fffffff;
   if (tiled && head_dim == 128) return launch_tiled<128>(a, G, workspace, workspace_bytes, s);
   if (tiled && head_dim == 64) return launch_tiled<64>(a, G, workspace, workspace_bytes, s);
@@ -978,7 +992,8 @@ extern "C" int64_t sf_tree_attention_workspace(int queries, int keys, int q_head
   if ((head_dim != 64 && head_dim != 128) || G > 16 ||
       static_cast<int64_t>(queries) * G > 0x3fffffff)
     return 0;
-  return tiled_workspace(tiled_plan(queries, keys, kv_heads, G, masked != 0), queries, q_heads, head_dim);
+  return tiled_workspace(tiled_plan(queries, keys, kv_heads, G, masked != 0), queries, q_heads,
+                         head_dim);
 }
 
 extern "C" int sf_tree_attention_split(const void* q, int64_t q_stride_token,
