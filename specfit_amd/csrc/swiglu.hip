@@ -673,6 +673,263 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
     down_body<R, 1, 1, NB, NT>(a, wk, tile, smem);
 }
 
+// -------------------------------------------------------- many-row experts --
+// Launches whose experts average many rows (a prompt: about T K / E rows per
+// expert) take a tiled GEMM instead of the streaming split above, which
+// re-reads its token rows for every 16 activation (32 output) columns and
+// feeds the matrix cores 32 x 32 per wavefront: at 128 rows per expert it was
+// bound by those re-reads (L2), not by the weights.
+//   Tile: up to 128 token rows x 128 weight rows (gate/up: 64 gate + 64 up
+//   rows of 64 columns; down: 128 output columns), k in blocks of 64.  Both
+//   operands pass through two LDS buffers (rows padded by 16 B: conflict-free
+//   16-byte fragment reads), loaded row-contiguously two blocks ahead into
+//   registers.  The 4 wavefronts are 2 (rows) x 2 (columns), 64 x 64 each.
+//   Passes: an expert's rows are cut into equal passes of at most 128 rows, in
+//   steps of 16, and an expert's workgroups share them (kPassSlots passes at a
+//   time), so 140 rows cost 2 x 80 rows and not 128 + 128.
+// Each output accumulates its k in ascending 32-steps like the streaming
+// split's KS = 1 form, so an expert of more than 32 rows has the same bits in
+// either kernel; experts of up to 32 rows take the streaming bodies here too.
+// Measured at (2048, 768), 128 experts, 2048 tokens with uniform routing:
+// gate/up 472 -> 250 us (412 TFLOP/s), down 276 -> 165 us.  What bounds it now
+// is the tiles' way from L2 into LDS, about 9 TB/s over the chip (each weight
+// tile is read once per pass, each token row once per 64 / 128 columns).
+constexpr int kWideK = 64;
+constexpr int kWideRowBytes = kWideK * 2 + 16;
+constexpr int kWideTile = 128 * kWideRowBytes;
+constexpr int kWideLds = 4 * kWideTile;  // two buffers of A and B
+constexpr int kPassSlots = 4;
+
+// 16 bytes at a uniform address plus a 32-bit byte offset.
+__device__ __forceinline__ sf_u32x4 ldv(const uint16_t* p, uint32_t byte_offset) {
+  return *(const __attribute__((address_space(1))) sf_u32x4*)(reinterpret_cast<const char*>(p) +
+                                                             byte_offset);
+}
+
+// acc[mt][n] of wavefront (wr, wc) = weight rows brow[n] .. of B times rows
+// 16 (2 mt + wr) .. of A over NB blocks of 64 k, transposed: a lane holds four
+// consecutive output columns 4 (l / 16) .. of token row l % 16 (8-byte
+// stores, one routing weight per tile).  This thread loads its 16-byte
+// piece tid % 8 of tile rows tid / 8 + 32 j: x + xo[j] of A, w[j] + wo of B
+// (x and w uniform, byte offsets).
+template <int MT, int NB>
+__device__ __forceinline__ void wide_gemm(const uint16_t* x, const uint32_t (&xo)[MT],
+                                          const uint16_t* const (&w)[4], uint32_t wo,
+                                          const int (&brow)[4], char* smem,
+                                          sf_f32x4 (&acc)[MT][4]) {
+  const int lane = threadIdx.x & (SF_WAVE - 1);
+  const int wr = threadIdx.x / SF_WAVE / 2;
+  const int st = (threadIdx.x / 8) * kWideRowBytes + (threadIdx.x % 8) * 16;
+  const int fr = (lane & 15) * kWideRowBytes + (lane >> 4) * 16;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[mt][n] = sf_f32x4{0.f, 0.f, 0.f, 0.f};
+  sf_u32x4 ra[2][MT], rb[2][4];
+  auto load = [&](int b, sf_u32x4 (&ar)[MT], sf_u32x4 (&br)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) br[j] = ldv(w[j] + b * kWideK, wo);
+#pragma unroll
+    for (int j = 0; j < MT; ++j) ar[j] = ldv(x + b * kWideK, xo[j]);
+  };
+  load(0, ra[0], rb[0]);
+  load(1, ra[1], rb[1]);
+  for (int b0 = 0; b0 < NB; b0 += 2) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      char* at = smem + i * 2 * kWideTile;
+      char* bt = at + kWideTile;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<sf_u32x4*>(bt + st + j * 32 * kWideRowBytes) = rb[i][j];
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        *reinterpret_cast<sf_u32x4*>(at + st + j * 32 * kWideRowBytes) = ra[i][j];
+      SF_SCHED_FENCE();
+      // Unconditional (the last two blocks load block NB - 1 again): a branch
+      // here would make the wait for the older loads a wait for all of them.
+      load(min(b0 + 2 + i, NB - 1), ra[i], rb[i]);
+      SF_SCHED_FENCE();
+      __syncthreads();  // block complete; the other buffer's reads are done
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        uint4 a[MT], f[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+          f[n] = *reinterpret_cast<const uint4*>(bt + brow[n] * kWideRowBytes + fr + 64 * s);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          a[mt] = *reinterpret_cast<const uint4*>(at + 16 * (2 * mt + wr) * kWideRowBytes + fr +
+                                                  64 * s);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int n = 0; n < 4; ++n) acc[mt][n] = mfma16(f[n], a[mt], acc[mt][n]);
+        SF_SCHED_FENCE();  // one k-step's fragments in registers at a time
+      }
+    }
+  }
+}
+
+// Gate/up of one pass (mp rows from permuted row base) and 64 columns c0.
+template <Resolve R, int MT, int NB>
+__device__ __forceinline__ void wide_gateup_pass(const SwigluArgs& a, const ExpertWork& wk, int base,
+                                                 int mp, int c0, char* smem) {
+  const int lane = threadIdx.x & (SF_WAVE - 1);
+  const int wave = threadIdx.x / SF_WAVE;
+  const int wr = wave / 2, wc = wave % 2;
+  const int trow = threadIdx.x / 8;
+  const uint32_t piece = 16 * (threadIdx.x % 8);
+  const uint16_t* wp[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)  // 64 gate rows, then 64 up rows
+    wp[j] = wk.w + static_cast<int64_t>(c0 + (j & 1) * 32 + (j >> 1) * a.I) * a.H;
+  uint32_t xo[MT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const int v = token_fetch<R>(a, base + min(32 * j + trow, mp - 1));
+    const uint32_t tok = R == Resolve::kDense ? v : v / a.top_k;
+    xo[j] = 2 * tok * static_cast<uint32_t>(a.row_stride) + piece;
+  }
+  const int brow[4] = {32 * wc, 32 * wc + 16, 64 + 32 * wc, 64 + 32 * wc + 16};
+  sf_f32x4 acc[MT][4];
+  wide_gemm<MT, NB>(a.hidden, xo, wp, 2 * trow * static_cast<uint32_t>(a.H) + piece, brow, smem,
+                    acc);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int row = 16 * (2 * mt + wr) + (lane & 15);
+    if (row >= mp) continue;
+    uint16_t* dst = a.act + static_cast<int64_t>(base + row) * a.I + c0 + 32 * wc + 4 * (lane >> 4);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      uint16_t v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float gb = sf_round_bf16(acc[mt][n][i]);
+        const float ub = sf_round_bf16(acc[mt][2 + n][i]);
+        const float sb = sf_round_bf16(sf_silu(gb));
+        v[i] = sf_f32_to_bf16(sb * ub);
+      }
+      *reinterpret_cast<uint2*>(dst + 16 * n) =
+          make_uint2(v[0] | static_cast<uint32_t>(v[1]) << 16,
+                     v[2] | static_cast<uint32_t>(v[3]) << 16);
+    }
+  }
+}
+
+template <int MT, int NB>
+__device__ __forceinline__ void wide_down_pass(const SwigluArgs& a, const ExpertWork& wk, int base,
+                                               int mp, int n0, char* smem) {
+  const int lane = threadIdx.x & (SF_WAVE - 1);
+  const int wave = threadIdx.x / SF_WAVE;
+  const int wr = wave / 2, wc = wave % 2;
+  const int trow = threadIdx.x / 8;
+  const uint32_t piece = 16 * (threadIdx.x % 8);
+  const uint16_t* wd = wk.w + 2 * static_cast<int64_t>(a.I) * a.H;
+  const uint16_t* wp[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) wp[j] = wd + static_cast<int64_t>(n0 + 32 * j) * a.I;
+  uint32_t xo[MT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j)
+    xo[j] = 2 * static_cast<uint32_t>(min(32 * j + trow, mp - 1)) * a.I + piece;
+  // Routing weights of this lane's rows, loaded while the product runs.
+  float rw[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int row = min(16 * (2 * mt + wr) + (lane & 15), mp - 1);
+    rw[mt] = a.route_w ? sf_bf16_to_f32(a.route_w[a.perm_pos[base + row]]) : 0.f;
+  }
+  const int brow[4] = {64 * wc, 64 * wc + 16, 64 * wc + 32, 64 * wc + 48};
+  sf_f32x4 acc[MT][4];
+  wide_gemm<MT, NB>(a.act + static_cast<int64_t>(base) * a.I, xo, wp,
+                    2 * trow * static_cast<uint32_t>(a.I) + piece, brow, smem, acc);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int row = 16 * (2 * mt + wr) + (lane & 15);
+    if (row >= mp) continue;
+    uint16_t* dst = a.out + static_cast<int64_t>(base + row) * a.H + n0 + 64 * wc + 4 * (lane >> 4);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      uint16_t v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float y = sf_round_bf16(acc[mt][n][i]);
+        if (a.route_w) y = y * rw[mt];
+        v[i] = sf_f32_to_bf16(y);
+      }
+      *reinterpret_cast<uint2*>(dst + 16 * n) =
+          make_uint2(v[0] | static_cast<uint32_t>(v[1]) << 16,
+                     v[2] | static_cast<uint32_t>(v[3]) << 16);
+    }
+  }
+}
+
+// Runs pass(base, mp, MT) for this workgroup's share of an expert's passes.
+template <typename Pass>
+__device__ __forceinline__ void wide_passes(const ExpertWork& wk, int slot, const Pass& pass) {
+  const int tiles = (wk.m + 15) / 16;
+  const int passes = (tiles + 7) / 8;
+  const int rows = (tiles + passes - 1) / passes * 16;
+  for (int64_t p0 = static_cast<int64_t>(slot) * rows; p0 < wk.m; p0 += kPassSlots * rows)
+    pass(wk.r0 + static_cast<int>(p0), min(rows, wk.m - static_cast<int>(p0)));
+}
+
+// Workgroup -> (expert j, tile, pass slot).  Consecutive workgroups run on
+// different XCDs.  One slot's column tiles of an expert stay on one XCD, whose
+// L2 then holds the slot's token rows; the slots are spread, so the many
+// passes of a popular expert do not queue on 32 CUs.  A slot's workgroups are
+// neighbours (the slots an expert has no pass for leave whole runs of
+// workgroups empty, not every fourth one, which would idle shader engines).
+// 2048 tokens, uniform / Zipf routing, us: one XCD per expert 412 / 555, no
+// placement 512 / 535.
+__device__ __forceinline__ void wide_place(int tiles, int& j, int& tile) {
+  const int group = blockIdx.x / (8 * tiles);
+  const int rest = blockIdx.x - group * 8 * tiles;
+  tile = rest >> 3;
+  j = group * 8 + ((rest - 2 * (tile * kPassSlots / tiles)) & 7);
+}
+
+template <Resolve R, int NBG>
+__global__ __launch_bounds__(kThreads, 2) void gateup_wide_kernel(const SwigluArgs a) {
+  __shared__ __attribute__((aligned(16))) char smem[kWideLds];
+  const int tiles = a.I / 16;
+  int j, tile;
+  wide_place(tiles, j, tile);
+  ExpertWork wk;
+  if (j >= a.n || !resolve<R>(a, j, wk)) return;
+  if (wk.m <= 16) return gateup_body<R, 1, 4, NBG, 2>(a, wk, tile, smem);
+  if (wk.m <= 32) return gateup_body<R, 1, 2, NBG, 2>(a, wk, tile, smem);
+  constexpr int NB = NBG * kBlockK / kWideK;
+  const int cols = tiles / kPassSlots;
+  const int c0 = tile % cols * 64;
+  wide_passes(wk, tile / cols, [&](int base, int mp) {
+    if (mp > 96) wide_gateup_pass<R, 4, NB>(a, wk, base, mp, c0, smem);
+    else if (mp > 64) wide_gateup_pass<R, 3, NB>(a, wk, base, mp, c0, smem);
+    else wide_gateup_pass<R, 2, NB>(a, wk, base, mp, c0, smem);
+  });
+}
+
+template <Resolve R, int NBD>
+__global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const SwigluArgs a) {
+  __shared__ __attribute__((aligned(16))) char smem[kWideLds];
+  const int tiles = a.H / 32;
+  int j, tile;
+  wide_place(tiles, j, tile);
+  ExpertWork wk;
+  if (j >= a.n || !resolve<R>(a, j, wk)) return;
+  if (wk.m <= 16) return down_body<R, 1, 4, NBD, 2>(a, wk, tile, smem);
+  if (wk.m <= 32) return down_body<R, 1, 2, NBD, 2>(a, wk, tile, smem);
+  constexpr int NB = NBD * kBlockK / kWideK;
+  const int cols = tiles / kPassSlots;
+  const int n0 = tile % cols * 128;
+  wide_passes(wk, tile / cols, [&](int base, int mp) {
+    if (mp > 96) wide_down_pass<4, NB>(a, wk, base, mp, n0, smem);
+    else if (mp > 64) wide_down_pass<3, NB>(a, wk, base, mp, n0, smem);
+    else wide_down_pass<2, NB>(a, wk, base, mp, n0, smem);
+  });
+}
+
 // ------------------------------------------------ generic (any shape) path --
 // One workgroup per expert; plain fp32 loops in ascending k.  Used for shapes
 // the MFMA tiling does not cover (tiny test models); same rounding points.
@@ -747,6 +1004,18 @@ int launch_mfma(const SwigluArgs& a, int groups, hipStream_t s) {
   return SF_OK;
 }
 
+template <Resolve R, int NBG, int NBD>
+int launch_wide(const SwigluArgs& a, int groups, hipStream_t s) {
+  const long long slots = (static_cast<long long>(groups) + 7) / 8 * 8;
+  const long long g1 = slots * (a.I / 16), g2 = slots * (a.H / 32);
+  if (g1 > 0x7fffffffLL || g2 > 0x7fffffffLL) return SF_ERR_UNSUPPORTED_SHAPE;
+  gateup_wide_kernel<R, NBG><<<dim3(static_cast<unsigned>(g1)), dim3(kThreads), 0, s>>>(a);
+  SF_LAUNCH_CHECK();
+  down_wide_kernel<R, NBD><<<dim3(static_cast<unsigned>(g2)), dim3(kThreads), 0, s>>>(a);
+  SF_LAUNCH_CHECK();
+  return SF_OK;
+}
+
 // Tile width.  A narrow launch (8 activation columns per gate/up workgroup,
 // 16 output columns per down workgroup) has twice the workgroups of a wide
 // one (16 / 32), so a launch of few small experts covers more CUs; each of
@@ -777,11 +1046,32 @@ int launch_width(const SwigluArgs& a, int groups, int max_rows, hipStream_t s) {
   return launch_class<R, 2, NBG, NBD>(a, groups, max_rows, s);
 }
 
+// The many-row kernels run where an expert may need a second pass of the
+// streaming split (above 128 rows), and for 65..128 rows where the launch has
+// enough of their larger tiles: from 8 experts at I = 768, 4 at I = 1536 (a
+// launch that leaves most CUs without a tile waits for one workgroup's whole
+// k loop, ~42 us).  Streaming / many-row, us, (H, I) = (2048, 768), experts
+// of 100 rows: 4: 29 / 47, 8: 49 / 48, 12: 68 / 58, 24: 116 / 82, 48: 209 /
+// 140; of 400 rows: 1: 85 / 45, 8: 159 / 73, 48: 751 / 332; (4096, 1536), 100
+// rows: 2: 47 / 81, 4: 86 / 84, 8: 138 / 93, 32: 525 / 272.  Slot-table
+// launches (T bounds the rows; most experts have fewer) at 128 experts,
+// uniform routing: T = 65: 243 / 214, 256: 271 / 230, 1024: 436 / 285, 2048:
+// 757 / 397; Zipf: T = 100: 118 / 127, 256: 209 / 164, 2048: 980 / 474.
+bool wide_launch(const SwigluArgs& a, int groups, int max_rows, long long tokens) {
+  if (max_rows <= 64 || tokens * a.row_stride >= (1ll << 31)) return false;  // 32-bit byte offsets
+  return max_rows > 128 || groups * static_cast<long long>(a.I) >= 8 * 768;
+}
+
 // max_rows bounds the rows of any expert of the launch; it picks the row
-// class of the build.
+// class of the build.  tokens: rows of a.hidden.
 template <Resolve R>
-int launch(const SwigluArgs& a, int groups, Shape shape, int max_rows, hipStream_t s) {
+int launch(const SwigluArgs& a, int groups, Shape shape, int max_rows, long long tokens,
+           hipStream_t s) {
   if (groups <= 0) return SF_OK;
+  if (wide_launch(a, groups, max_rows, tokens)) {
+    if (shape == Shape::k2048x768) return launch_wide<R, 8, 3>(a, groups, s);
+    if (shape == Shape::k4096x1536) return launch_wide<R, 16, 6>(a, groups, s);
+  }
   if (shape == Shape::k2048x768) return launch_width<R, 8, 3>(a, groups, max_rows, s);
   if (shape == Shape::k4096x1536) return launch_width<R, 16, 6>(a, groups, max_rows, s);
   gateup_generic_kernel<R><<<dim3(groups), dim3(kThreads), 0, s>>>(a);
@@ -853,7 +1143,7 @@ extern "C" int sf_grouped_swiglu(const void* hidden, const int32_t* perm_pos,
         a.rows[i] = expert_row_count[base + i];
       }
     }
-    rc = launch<Resolve::kList>(a, a.n, shape, max_rows, s);
+    rc = launch<Resolve::kList>(a, a.n, shape, max_rows, tokens, s);
     if (rc) return rc;
   }
   return SF_OK;
@@ -886,7 +1176,7 @@ int table_launch(const void* hidden, const int32_t* perm_pos, const int32_t* off
   a.slot_of_expert = slot_of_expert;
   a.slot_base = static_cast<const uint16_t*>(slot_base);
   a.slot_stride = slot_stride_elems;
-  return launch<Resolve::kTable>(a, num_experts, shape, max_rows, stream);
+  return launch<Resolve::kTable>(a, num_experts, shape, max_rows, tokens, stream);
 }
 
 int check_table(int tokens, int top_k, int hidden_size, int intermediate_size, int num_experts,
@@ -1013,5 +1303,5 @@ extern "C" int sf_expert_swiglu(const void* rows, int m, int64_t row_stride,
   a.dense_m = m;
   a.n = 1;
   a.wptr[0] = reinterpret_cast<uint64_t>(packed_weights);
-  return launch<Resolve::kDense>(a, 1, shape, m, reinterpret_cast<hipStream_t>(stream));
+  return launch<Resolve::kDense>(a, 1, shape, m, m, reinterpret_cast<hipStream_t>(stream));
 }

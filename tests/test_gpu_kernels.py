@@ -341,6 +341,51 @@ def test_grouped_swiglu_qwen3_235b_shape(device):
     np.testing.assert_allclose(oracle.bf16_float(_bits(rows)), ref_rows, rtol=1.6e-2, atol=1.6e-2)
 
 
+@pytest.mark.parametrize("H,I", [(2048, 768), (4096, 1536)])
+def test_many_row_kernels_match_the_streaming_split(device, H, I):
+    """One launch of experts with row counts around every edge of the
+    many-row tiles (16-row steps, 64 / 96 / 128-row tiles, equal passes, the
+    pass slots) against each expert's rows in chunks of at most 128, which run
+    the streaming split: the same bits, as both add k in ascending 32-steps."""
+    counts = [1, 16, 17, 32, 33, 64, 65, 96, 97, 0, 128, 129, 160, 161, 257, 530]
+    E, T = len(counts), max(counts)
+    g = torch.Generator("cpu").manual_seed(H)
+    hidden = torch.randn(T, H, generator=g).to(torch.bfloat16).to(device)
+    slots = (torch.randn(E, 3 * H * I, generator=g) * 0.03).to(torch.bfloat16).to(device)
+    idx = torch.full((T, E), -1, dtype=torch.int64)
+    for e, m in enumerate(counts):  # expert e takes m tokens, spread over the batch
+        idx[torch.randperm(T, generator=g)[:m], e] = e
+    idx = idx.to(device)
+    plan = ops.dispatch(idx, E)
+    act = torch.empty((T * E, I), dtype=torch.bfloat16, device=device)
+    rows = torch.zeros((T * E, H), dtype=torch.bfloat16, device=device)
+    table = torch.arange(E, dtype=torch.int32, device=device)
+    ops.grouped_swiglu_table(hidden, plan, None, table, slots, H, I, act, rows, max_rows=T)
+    perm, offsets = plan.perm_pos.cpu(), plan.offsets.tolist()
+    for e, m in enumerate(counts):
+        tokens = (perm[offsets[e]:offsets[e + 1]].long() // E).to(device)
+        got = rows[offsets[e]:offsets[e + 1]]
+        for at in range(0, m, 128):
+            lo = max(0, min(at, m - 128)) if m > 128 else 0  # the last chunk overlaps: above 32 rows
+            hi = min(m, lo + 128)
+            want = ops.expert_swiglu(hidden[tokens[lo:hi]], slots[e], H, I)
+            assert torch.equal(got[lo:hi], want), (e, m, lo, hi)
+    # With routing weights: the unscaled rows times the weight, rounded once more.
+    weights = torch.rand(T * E, generator=g).to(torch.bfloat16).to(device)
+    scaled = torch.zeros_like(rows)
+    ops.grouped_swiglu_table(hidden, plan, weights, table, slots, H, I, act, scaled, max_rows=T)
+    n = offsets[E]
+    want = (rows[:n].float() * weights[plan.perm_pos[:n].long()].float()[:, None]).to(torch.bfloat16)
+    assert torch.equal(scaled[:n], want)
+    # A single expert of many rows takes the same kernels.
+    x = torch.randn(300, H, generator=g).to(torch.bfloat16).to(device)
+    padded = torch.zeros(300, H + 8, dtype=torch.bfloat16, device=device)
+    padded[:, :H] = x
+    y = ops.expert_swiglu(padded[:, :H], slots[2], H, I)
+    for lo in (0, 128, 172):
+        assert torch.equal(y[lo:lo + 128], ops.expert_swiglu(x[lo:lo + 128], slots[2], H, I))
+
+
 @pytest.mark.parametrize("H,I,m", [(4, 3, 2), (32, 16, 5), (96, 64, 70), (2048, 768, 48),
                                    (2048, 768, 130), (4096, 1536, 20), (4096, 1536, 70)])
 def test_expert_swiglu_generic_and_mfma_paths(device, H, I, m):
