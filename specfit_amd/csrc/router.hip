@@ -42,6 +42,14 @@ __device__ __forceinline__ float dot8_acc(uint4 hv, uint4 wv, float acc) {
   return acc;
 }
 
+typedef unsigned int router_u32x4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes at a uniform address plus a 32-bit byte offset.
+__device__ __forceinline__ router_u32x4 router_ld16(const uint16_t* p, uint32_t byte_offset) {
+  return *(const __attribute__((address_space(1))) router_u32x4*)(
+      reinterpret_cast<const char*>(p) + byte_offset);
+}
+
 // Softmax + top-k + renorm over s_logit[0..E) by one wavefront.  Lane l
 // reads only experts l, l+64, ... of s_logit.  Each top-k round takes the
 // wave maximum of the unselected probabilities and the lowest expert id
@@ -181,6 +189,114 @@ __global__ __launch_bounds__(kLogitWaves * SF_WAVE) void router_logits_kernel(
     logits[static_cast<size_t>(t) * E + e] = sf_f32_to_bf16(a);
 }
 
+// Many tokens: a wavefront takes 8 tokens x 8 experts, so a chunk's 16 loads
+// and 128 unpacking instructions serve 512 multiply-adds (the 2 x 4 tile
+// above: 6 loads and 48 for 64), and the 64 sums of the tile go through one
+// transposed butterfly: at distance d a lane keeps the half of its sums whose
+// index has the lane's bit d and adds the partner's copy of those (about 3
+// instructions a logit instead of 11), ending with logit l of the tile in
+// lane l.  Every addition has the same two operands as in sf_wave_sum, so the
+// bits are the same.  Bound by the vector ALU (2048 of its 2754 instructions
+// per tile are the multiply-adds of H = 2048).  Any H of whole chunk rounds
+// (512 elements).
+// Taken from 32768 logits on, where its tiles fill the chip: both kernels of
+// the call at E = 128, small / large tile, us: H = 2048, T = 128: 9.5 / 12.4,
+// 256: 13.0 / 12.6, 512: 20.1 / 12.9, 2048: 57.5 / 26.6; H = 4096, T = 192:
+// 15.5 / 18.8, 256: 18.5 / 19.2, 384: 24.5 / 19.5, 2048: 101 / 42.7.
+constexpr int kManyTile = 8;  // tokens and experts of a wavefront
+constexpr long long kManyLogits = 32768;
+
+template <int CTRL>
+__device__ __forceinline__ float butterfly_pair(float even, float odd, bool bit) {
+  const float keep = bit ? odd : even;
+  const float send = bit ? even : odd;
+  return keep + sf_dpp<CTRL>(send);
+}
+
+__device__ __forceinline__ float unpack_lo(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float unpack_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+
+__global__ __launch_bounds__(kLogitWaves * SF_WAVE, 2) void router_logits_many_kernel(
+    const uint16_t* __restrict__ hidden, const uint16_t* __restrict__ wr, int T, int H, int E,
+    uint16_t* __restrict__ logits) {
+  const int lane = threadIdx.x & (SF_WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SF_WAVE);
+  const int t0 = blockIdx.x * kManyTile;
+  const int e0 = (blockIdx.y * kLogitWaves + wave) * kManyTile;
+  if (e0 >= E) return;  // wave-uniform; the kernel has no block barrier
+  uint32_t ho[kManyTile], wo[kManyTile];  // byte offsets: T H and E H stay below 2^31
+#pragma unroll
+  for (int i = 0; i < kManyTile; ++i) {
+    ho[i] = 2u * min(t0 + i, T - 1) * H + 16 * lane;
+    wo[i] = 2u * min(e0 + i, E - 1) * H + 16 * lane;
+  }
+  router_u32x4 h[kManyTile], w[kManyTile];
+  auto load = [&](int k) {  // the lane's chunk at element k + 8 lane of every row
+#pragma unroll
+    for (int i = 0; i < kManyTile; ++i) {
+      h[i] = router_ld16(hidden + k, ho[i]);
+      w[i] = router_ld16(wr + k, wo[i]);
+    }
+  };
+  float acc[kManyTile * kManyTile];
+#pragma unroll
+  for (int v = 0; v < kManyTile * kManyTile; ++v) acc[v] = 0.0f;
+  constexpr int kStep = 8 * SF_WAVE;
+  load(0);
+  for (int k = 0; k < H; k += kStep) {
+    router_u32x4 hc[kManyTile], wc[kManyTile];
+#pragma unroll
+    for (int i = 0; i < kManyTile; ++i) {
+      hc[i] = h[i];
+      wc[i] = w[i];
+    }
+    load(min(k + kStep, H - kStep));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        float hf[kManyTile], wf[kManyTile];
+#pragma unroll
+        for (int i = 0; i < kManyTile; ++i) {
+          hf[i] = half ? unpack_hi(hc[i][q]) : unpack_lo(hc[i][q]);
+          wf[i] = half ? unpack_hi(wc[i][q]) : unpack_lo(wc[i][q]);
+        }
+#pragma unroll
+        for (int t = 0; t < kManyTile; ++t)
+#pragma unroll
+          for (int e = 0; e < kManyTile; ++e)
+            acc[kManyTile * t + e] = __builtin_fmaf(hf[t], wf[e], acc[kManyTile * t + e]);
+      }
+    }
+  }
+  // Distances 1, 2, 4, 8, 16, 32 over sum-index bits 0 .. 5.
+#pragma unroll
+  for (int p = 0; p < 32; ++p) acc[p] = butterfly_pair<0xB1>(acc[2 * p], acc[2 * p + 1], lane & 1);
+#pragma unroll
+  for (int p = 0; p < 16; ++p) acc[p] = butterfly_pair<0x4E>(acc[2 * p], acc[2 * p + 1], lane & 2);
+#pragma unroll
+  for (int p = 0; p < 8; ++p) {  // lane ^ 4 = the half-row mirror (^ 7) of ^ 3
+    const bool bit = lane & 4;
+    const float keep = bit ? acc[2 * p + 1] : acc[2 * p];
+    const float send = bit ? acc[2 * p] : acc[2 * p + 1];
+    acc[p] = keep + sf_dpp<0x141>(sf_dpp<0x1B>(send));
+  }
+#pragma unroll
+  for (int p = 0; p < 4; ++p) acc[p] = butterfly_pair<0x128>(acc[2 * p], acc[2 * p + 1], lane & 8);
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const auto r = __builtin_amdgcn_permlane16_swap(
+        __float_as_int(acc[2 * p]), __float_as_int(acc[2 * p + 1]), false, false);
+    acc[p] = __int_as_float(r[0]) + __int_as_float(r[1]);
+  }
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(acc[0]), __float_as_int(acc[1]),
+                                                  false, false);
+  const float total = __int_as_float(r[0]) + __int_as_float(r[1]);
+  const int t = t0 + lane / kManyTile;
+  const int e = e0 + lane % kManyTile;
+  if (t < T && e < E) logits[static_cast<size_t>(t) * E + e] = sf_f32_to_bf16(total);
+}
+
 constexpr int kSelectWaves = 4;
 
 template <int J>  // experts per lane: E <= 64 * J
@@ -257,7 +373,11 @@ extern "C" int sf_router_topk(const void* hidden, const void* router_weight,
                        (hidden_size % 8 == 0);
   const int nchunks = (hidden_size + 7) / 8;
   const int per_lane = (nchunks + SF_WAVE - 1) / SF_WAVE;
-  if (aligned && per_lane <= 16) {
+  const bool many = aligned && hidden_size % (8 * SF_WAVE) == 0 &&
+                    static_cast<long long>(tokens) * num_experts >= kManyLogits &&
+                    static_cast<long long>(tokens) * hidden_size < (1ll << 31) &&
+                    static_cast<long long>(num_experts) * hidden_size < (1ll << 31);
+  if (aligned && (many || per_lane <= 16)) {
     int tt = 1, epw = 1;
     auto logits_launch = [&](auto kernel, int tile_tokens, int tile_experts) {
       tt = tile_tokens;
@@ -266,7 +386,9 @@ extern "C" int sf_router_topk(const void* hidden, const void* router_weight,
       dim3 grid((tokens + tt - 1) / tt, (num_experts + per_block - 1) / per_block);
       kernel<<<grid, dim3(kLogitWaves * SF_WAVE), 0, s>>>(h, w, tokens, hidden_size, num_experts, lg);
     };
-    if (per_lane <= 1)
+    if (many)
+      logits_launch(router_logits_many_kernel, kManyTile, kManyTile);
+    else if (per_lane <= 1)
       logits_launch(router_logits_kernel<1>, LogitTile<1>::tokens, LogitTile<1>::experts);
     else if (per_lane <= 2)
       logits_launch(router_logits_kernel<2>, LogitTile<2>::tokens, LogitTile<2>::experts);

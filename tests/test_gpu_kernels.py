@@ -69,6 +69,15 @@ def test_router_bitexact_other_shapes(device, T, H, E, K, renorm):
     _router_case(device, T, H, E, K, renorm, 21)
 
 
+# The many-token tile: its first sizes, remainders of its 8 tokens and 8
+# experts, one and many chunk rounds, and widths past the small tile's.
+@pytest.mark.parametrize("T,H,E,K", [(255, 2048, 128, 8), (256, 2048, 128, 8), (257, 512, 128, 8),
+                                     (331, 1024, 99, 8), (600, 4096, 57, 4), (1025, 2048, 32, 8),
+                                     (260, 9216, 128, 8), (520, 1536, 256, 32)])
+def test_router_bitexact_many_tokens(device, T, H, E, K):
+    _router_case(device, T, H, E, K, True, 33)
+
+
 def test_router_ties_resolve_to_lower_id(device):
     h = torch.zeros(3, 256, dtype=torch.bfloat16)
     w = _randn_bf16((16, 256), 4, 0.02)
