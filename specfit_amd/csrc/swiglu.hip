@@ -679,25 +679,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
 // re-reads its token rows for every 16 activation (32 output) columns and
 // feeds the matrix cores 32 x 32 per wavefront: at 128 rows per expert it was
 // bound by those re-reads (L2), not by the weights.
-//   Tile: up to 128 token rows x 128 weight rows (gate/up: 64 gate + 64 up
+//   Tile: up to 160 token rows x 128 weight rows (gate/up: 64 gate + 64 up
 //   rows of 64 columns; down: 128 output columns), k in blocks of 64.  Both
-//   operands pass through two LDS buffers (rows padded by 16 B: conflict-free
-//   16-byte fragment reads), loaded row-contiguously two blocks ahead into
-//   registers.  The 4 wavefronts are 2 (rows) x 2 (columns), 64 x 64 each.
-//   Passes: an expert's rows are cut into equal passes of at most 128 rows, in
+//   operands pass through LDS (rows padded by 16 B), loaded row-contiguously
+//   two blocks ahead into registers; two workgroups share a CU, so one's
+//   barriers hide behind the other's matrix work.  The 4 wavefronts are 2
+//   (rows) x 2 (columns), up to 80 x 64 each.
+//   Passes: an expert's rows are cut into equal passes of at most 160 rows, in
 //   steps of 16, and an expert's workgroups share them (kPassSlots passes at a
-//   time), so 140 rows cost 2 x 80 rows and not 128 + 128.
+//   time).  At 128 rows per expert on average most experts then need one
+//   pass and read their weights once: 416 us for both kernels with passes of
+//   up to 128 rows (and two LDS buffers), 364 with 160, 368 with 192.
 // Each output accumulates its k in ascending 32-steps like the streaming
 // split's KS = 1 form, so an expert of more than 32 rows has the same bits in
 // either kernel; experts of up to 32 rows take the streaming bodies here too.
 // Measured at (2048, 768), 128 experts, 2048 tokens with uniform routing:
-// gate/up 472 -> 250 us (412 TFLOP/s), down 276 -> 165 us.  What bounds it now
-// is the tiles' way from L2 into LDS, about 9 TB/s over the chip (each weight
-// tile is read once per pass, each token row once per 64 / 128 columns).
+// both kernels 748 -> 364 us (425 TFLOP/s; the weights, 1.2 GB, stream at 3.3
+// TB/s).  What bounds it: memory latency under load, with two 64-k blocks in
+// flight per workgroup (matrix cores 26% busy, LDS 45%); 256 B instead of
+// 128 B per row and load gave no more.
 constexpr int kWideK = 64;
 constexpr int kWideRowBytes = kWideK * 2 + 16;
-constexpr int kWideTile = 128 * kWideRowBytes;
-constexpr int kWideLds = 4 * kWideTile;  // two buffers of A and B
+constexpr int kPassRows = 160;
+constexpr int kWideLds = (kPassRows + 128) * kWideRowBytes;  // A, then B
 constexpr int kPassSlots = 4;
 
 // 16 bytes at a uniform address plus a 32-bit byte offset.
@@ -734,23 +738,22 @@ __device__ __forceinline__ void wide_gemm(const uint16_t* x, const uint32_t (&xo
   };
   load(0, ra[0], rb[0]);
   load(1, ra[1], rb[1]);
+  char* bt = smem + kPassRows * kWideRowBytes;
   for (int b0 = 0; b0 < NB; b0 += 2) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      char* at = smem + i * 2 * kWideTile;
-      char* bt = at + kWideTile;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         *reinterpret_cast<sf_u32x4*>(bt + st + j * 32 * kWideRowBytes) = rb[i][j];
 #pragma unroll
       for (int j = 0; j < MT; ++j)
-        *reinterpret_cast<sf_u32x4*>(at + st + j * 32 * kWideRowBytes) = ra[i][j];
+        *reinterpret_cast<sf_u32x4*>(smem + st + j * 32 * kWideRowBytes) = ra[i][j];
       SF_SCHED_FENCE();
       // Unconditional (the last two blocks load block NB - 1 again): a branch
       // here would make the wait for the older loads a wait for all of them.
       load(min(b0 + 2 + i, NB - 1), ra[i], rb[i]);
       SF_SCHED_FENCE();
-      __syncthreads();  // block complete; the other buffer's reads are done
+      __syncthreads();  // the block is complete
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         uint4 a[MT], f[4];
@@ -759,7 +762,7 @@ __device__ __forceinline__ void wide_gemm(const uint16_t* x, const uint32_t (&xo
           f[n] = *reinterpret_cast<const uint4*>(bt + brow[n] * kWideRowBytes + fr + 64 * s);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
-          a[mt] = *reinterpret_cast<const uint4*>(at + 16 * (2 * mt + wr) * kWideRowBytes + fr +
+          a[mt] = *reinterpret_cast<const uint4*>(smem + 16 * (2 * mt + wr) * kWideRowBytes + fr +
                                                   64 * s);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
@@ -767,6 +770,7 @@ __device__ __forceinline__ void wide_gemm(const uint16_t* x, const uint32_t (&xo
           for (int n = 0; n < 4; ++n) acc[mt][n] = mfma16(f[n], a[mt], acc[mt][n]);
         SF_SCHED_FENCE();  // one k-step's fragments in registers at a time
       }
+      __syncthreads();  // its reads are done
     }
   }
 }
@@ -869,7 +873,7 @@ __device__ __forceinline__ void wide_down_pass(const SwigluArgs& a, const Expert
 template <typename Pass>
 __device__ __forceinline__ void wide_passes(const ExpertWork& wk, int slot, const Pass& pass) {
   const int tiles = (wk.m + 15) / 16;
-  const int passes = (tiles + 7) / 8;
+  const int passes = (tiles + kPassRows / 16 - 1) / (kPassRows / 16);
   const int rows = (tiles + passes - 1) / passes * 16;
   for (int64_t p0 = static_cast<int64_t>(slot) * rows; p0 < wk.m; p0 += kPassSlots * rows)
     pass(wk.r0 + static_cast<int>(p0), min(rows, wk.m - static_cast<int>(p0)));
@@ -881,8 +885,8 @@ __device__ __forceinline__ void wide_passes(const ExpertWork& wk, int slot, cons
 // passes of a popular expert do not queue on 32 CUs.  A slot's workgroups are
 // neighbours (the slots an expert has no pass for leave whole runs of
 // workgroups empty, not every fourth one, which would idle shader engines).
-// 2048 tokens, uniform / Zipf routing, us: one XCD per expert 412 / 555, no
-// placement 512 / 535.
+// 2048 tokens, uniform / Zipf routing, us: 364 / 474; one XCD per expert 370 /
+// 508.
 __device__ __forceinline__ void wide_place(int tiles, int& j, int& tile) {
   const int group = blockIdx.x / (8 * tiles);
   const int rest = blockIdx.x - group * 8 * tiles;
@@ -904,7 +908,8 @@ __global__ __launch_bounds__(kThreads, 2) void gateup_wide_kernel(const SwigluAr
   const int cols = tiles / kPassSlots;
   const int c0 = tile % cols * 64;
   wide_passes(wk, tile / cols, [&](int base, int mp) {
-    if (mp > 96) wide_gateup_pass<R, 4, NB>(a, wk, base, mp, c0, smem);
+    if (mp > 128) wide_gateup_pass<R, 5, NB>(a, wk, base, mp, c0, smem);
+    else if (mp > 96) wide_gateup_pass<R, 4, NB>(a, wk, base, mp, c0, smem);
     else if (mp > 64) wide_gateup_pass<R, 3, NB>(a, wk, base, mp, c0, smem);
     else wide_gateup_pass<R, 2, NB>(a, wk, base, mp, c0, smem);
   });
@@ -924,7 +929,8 @@ __global__ __launch_bounds__(kThreads, 2) void down_wide_kernel(const SwigluArgs
   const int cols = tiles / kPassSlots;
   const int n0 = tile % cols * 128;
   wide_passes(wk, tile / cols, [&](int base, int mp) {
-    if (mp > 96) wide_down_pass<4, NB>(a, wk, base, mp, n0, smem);
+    if (mp > 128) wide_down_pass<5, NB>(a, wk, base, mp, n0, smem);
+    else if (mp > 96) wide_down_pass<4, NB>(a, wk, base, mp, n0, smem);
     else if (mp > 64) wide_down_pass<3, NB>(a, wk, base, mp, n0, smem);
     else wide_down_pass<2, NB>(a, wk, base, mp, n0, smem);
   });
@@ -1055,8 +1061,8 @@ int launch_width(const SwigluArgs& a, int groups, int max_rows, hipStream_t s) {
 // 140; of 400 rows: 1: 85 / 45, 8: 159 / 73, 48: 751 / 332; (4096, 1536), 100
 // rows: 2: 47 / 81, 4: 86 / 84, 8: 138 / 93, 32: 525 / 272.  Slot-table
 // launches (T bounds the rows; most experts have fewer) at 128 experts,
-// uniform routing: T = 65: 243 / 214, 256: 271 / 230, 1024: 436 / 285, 2048:
-// 757 / 397; Zipf: T = 100: 118 / 127, 256: 209 / 164, 2048: 980 / 474.
+// uniform routing: T = 65: 243 / 214, 256: 271 / 233, 1024: 436 / 285, 2048:
+// 757 / 364; Zipf: T = 100: 118 / 127, 256: 209 / 169, 2048: 980 / 474.
 bool wide_launch(const SwigluArgs& a, int groups, int max_rows, long long tokens) {
   if (max_rows <= 64 || tokens * a.row_stride >= (1ll << 31)) return false;  // 32-bit byte offsets
   return max_rows > 128 || groups * static_cast<long long>(a.I) >= 8 * 768;
