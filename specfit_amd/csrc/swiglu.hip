@@ -880,18 +880,20 @@ __device__ __forceinline__ void wide_passes(const ExpertWork& wk, int slot, cons
 }
 
 // Workgroup -> (expert j, tile, pass slot).  Consecutive workgroups run on
-// different XCDs.  One slot's column tiles of an expert stay on one XCD, whose
-// L2 then holds the slot's token rows; the slots are spread, so the many
-// passes of a popular expert do not queue on 32 CUs.  A slot's workgroups are
-// neighbours (the slots an expert has no pass for leave whole runs of
-// workgroups empty, not every fourth one, which would idle shader engines).
-// 2048 tokens, uniform / Zipf routing, us: 364 / 474; one XCD per expert 370 /
-// 508.
+// different XCDs.  Half the column tiles of a pass slot stay on one XCD, whose
+// L2 then serves the slot's token rows to all of them, and an expert's eighths
+// are spread over the XCDs, so neither a popular expert's passes nor a small
+// expert's weights queue on 32 CUs.  A slot's workgroups are neighbours (the
+// slots an expert has no pass for leave whole runs of workgroups empty, not
+// every fourth one, which would idle shader engines: 876 us for 2048 tokens).
+// 2048 tokens, uniform / Zipf routing, us: 365 / 469; a slot per XCD 371 /
+// 474; an expert per XCD 370 / 508.  512 tokens: 276 / 201, 286 / 207, 275 /
+// 257.
 __device__ __forceinline__ void wide_place(int tiles, int& j, int& tile) {
   const int group = blockIdx.x / (8 * tiles);
   const int rest = blockIdx.x - group * 8 * tiles;
   tile = rest >> 3;
-  j = group * 8 + ((rest - 2 * (tile * kPassSlots / tiles)) & 7);
+  j = group * 8 + ((rest - tile * 8 / tiles) & 7);
 }
 
 template <Resolve R, int NBG>
@@ -1061,10 +1063,13 @@ int launch_width(const SwigluArgs& a, int groups, int max_rows, hipStream_t s) {
 // 140; of 400 rows: 1: 85 / 45, 8: 159 / 73, 48: 751 / 332; (4096, 1536), 100
 // rows: 2: 47 / 81, 4: 86 / 84, 8: 138 / 93, 32: 525 / 272.  Slot-table
 // launches (T bounds the rows; most experts have fewer) at 128 experts,
-// uniform routing: T = 65: 243 / 214, 256: 271 / 233, 1024: 436 / 285, 2048:
-// 757 / 364; Zipf: T = 100: 118 / 127, 256: 209 / 169, 2048: 980 / 474.
-bool wide_launch(const SwigluArgs& a, int groups, int max_rows, long long tokens) {
+// uniform routing: T = 65: 244 / 214, 256: 272 / 232, 1024: 425 / 287, 2048:
+// 751 / 365; Zipf: T = 100: 118 / 120, 256: 209 / 169, 2048: 975 / 469.
+// A slot-table launch of few experts with up to 32 rows on average streams:
+// 32 experts of (4096, 1536), T = 100: 263 / 268, 128: 268 / 280.
+bool wide_launch(const SwigluArgs& a, Resolve r, int groups, int max_rows, long long tokens) {
   if (max_rows <= 64 || tokens * a.row_stride >= (1ll << 31)) return false;  // 32-bit byte offsets
+  if (r == Resolve::kTable && groups < 64 && tokens * a.top_k <= 32ll * groups) return false;
   return max_rows > 128 || groups * static_cast<long long>(a.I) >= 8 * 768;
 }
 
@@ -1074,7 +1079,7 @@ template <Resolve R>
 int launch(const SwigluArgs& a, int groups, Shape shape, int max_rows, long long tokens,
            hipStream_t s) {
   if (groups <= 0) return SF_OK;
-  if (wide_launch(a, groups, max_rows, tokens)) {
+  if (wide_launch(a, R, groups, max_rows, tokens)) {
     if (shape == Shape::k2048x768) return launch_wide<R, 8, 3>(a, groups, s);
     if (shape == Shape::k4096x1536) return launch_wide<R, 16, 6>(a, groups, s);
   }
