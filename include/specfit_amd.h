@@ -31,7 +31,8 @@
  *                        (slot.tensor.copy_(pinned_source, non_blocking=True))
  *   sf_expert_decode     the same copy when the transfer moves an
  *                        exponent-coded record (decoded into the slot)
- *   sf_tree_attention    the attention of the verification forward:
+ *   sf_tree_attention, sf_tree_attention_split
+ *                        the attention of the verification forward:
  *                        eagle3_tree.py:1202-1240 runs the target with
  *                        Eagle3DraftTree.verification_attention_mask
  *                        (eagle3_types.py:450-473); each Qwen3 attention layer
