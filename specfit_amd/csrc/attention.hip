@@ -319,9 +319,17 @@ struct TiledArgs {
   int row_tiles;     // of 32 WR rows
   int splits;
   int split_keys;    // keys of one split, a multiple of 64 * 4 / WR
+  float c;           // |scale| log2(e): scores to log2 units
   float* part_acc;   // [splits][Hkv][rows][D], splits > 1 only
-  float2* part_ml;   // [splits][Hkv][rows] (max in log2 units, sum)
+  float2* part_ml;   // [splits][Hkv][rows] (max of the unscaled scores, sum)
 };
+
+// p = exp2(s c - m c) is one fused multiply-add per score, but it subtracts
+// the rounded m c from the exact s c.  Up to this |m c| the difference at the
+// row's maximum is at most 2^-13, far below the rounding of P to bf16 (2^-9);
+// at 2^31 it would be 128, and the row's sum 0 or infinite.  A wavefront with
+// a row past it subtracts before it scales.
+constexpr float kFusedMax = 4096.f;
 
 // Rows padded so the fragment reads spread over the banks: 16 B for the
 // 16-byte reads of K (16 consecutive rows), 32 B for the transposed reads of
@@ -403,10 +411,11 @@ __device__ __forceinline__ uint32_t mask_word(const uint8_t* row, int key, int S
   return w;
 }
 
-// One more (max, sum, accumulator) state, weighted against the maximum M.
-__device__ __forceinline__ void add_state(float m, float l, const float4& v, float M, float& sum,
-                                          float (&o)[4]) {
-  const float f = __builtin_amdgcn_exp2f(m - M);
+// One more (max, sum, accumulator) state, weighted against the maximum M of
+// the unscaled scores (subtracted before scaling, see kFusedMax).
+__device__ __forceinline__ void add_state(float m, float l, const float4& v, float M, float c,
+                                          float& sum, float (&o)[4]) {
+  const float f = __builtin_amdgcn_exp2f((m - M) * c);
   sum = __builtin_fmaf(l, f, sum);
   o[0] = __builtin_fmaf(v.x, f, o[0]);
   o[1] = __builtin_fmaf(v.y, f, o[1]);
@@ -468,7 +477,7 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
     for (int s = 0; s < kSteps; ++s)
       qf[s] = __builtin_bit_cast(sf_bf16x8, ld16(qr + 16 * s) ^ flip);
   }
-  const float c = fabsf(a.scale) * 1.44269504088896341f;  // log2 units
+  const float c = t.c;
 
   // Keys: [begin, end) for the workgroup; the wavefront's rows see none from
   // wave_end on, and all of them see the keys below wave_full.
@@ -589,8 +598,7 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
         for (int kt = 0; kt < 2; ++kt) mx[kt] = max_raw(mx[kt], s[kt][i]);
       const float mnew = fmaxf(m, half_max(max_raw(mx[0], mx[1])));
       if (__any(mnew > m)) {
-        const float alpha =
-            m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m * c - mnew * c);
+        const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mnew) * c);
         l *= alpha;
 #pragma unroll
         for (int dt = 0; dt < kDt; ++dt)
@@ -598,7 +606,15 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
           for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
         m = mnew;
       }
-      const float base = m == -INFINITY ? 0.f : -(m * c);
+      float base = m == -INFINITY ? 0.f : -(m * c);
+      if (__any(fabsf(base) > kFusedMax)) {
+        const float top = m == -INFINITY ? 0.f : m;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[kt][i] -= top;
+        base = 0.f;
+      }
       uint32_t pk[2][8];
       float sum[2] = {0.f, 0.f};
 #pragma unroll
@@ -631,14 +647,13 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
     if (WR != 4) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // tile reused
   }
   l = half_sum(l);
-  const float mlog = m == -INFINITY ? -INFINITY : m * c;
 
   const int64_t part_row = (static_cast<int64_t>(split) * a.Hkv + h) * t.rows;
   if (WR == 4) {
     if (row >= t.rows) return;
     if (t.splits > 1) {
-      if (hf == 0) t.part_ml[part_row + row] = make_float2(mlog, l);
-      if (mlog == -INFINITY) return;  // never read
+      if (hf == 0) t.part_ml[part_row + row] = make_float2(m, l);
+      if (m == -INFINITY) return;  // never read
       float* o = t.part_acc + (part_row + row) * D + 4 * hf;
 #pragma unroll
       for (int dt = 0; dt < kDt; ++dt)
@@ -663,7 +678,7 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
     float* sml = sacc + kWk * kRows * L::orow;                   // [kWk][kRows][2]
     const int lrow = kg * kRows + 32 * (wave % WR) + col;
     if (hf == 0) {
-      sml[2 * lrow] = mlog;
+      sml[2 * lrow] = m;
       sml[2 * lrow + 1] = l;
     }
 #pragma unroll
@@ -686,8 +701,8 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
         const float wm = sml[2 * (w * kRows + lr)];
         if (wm == -INFINITY) continue;
         add_state(wm, sml[2 * (w * kRows + lr) + 1],
-                  *reinterpret_cast<const float4*>(sacc + (w * kRows + lr) * L::orow + d), M, sum,
-                  o);
+                  *reinterpret_cast<const float4*>(sacc + (w * kRows + lr) * L::orow + d), M, c,
+                  sum, o);
       }
       if (t.splits > 1) {
         if (d == 0) t.part_ml[part_row + r] = make_float2(M, sum);
@@ -741,7 +756,7 @@ __global__ __launch_bounds__(kTileThreads) void tree_attention_merge_kernel(cons
 #pragma unroll
   for (int j = 0; j < kMergeDepth; ++j) {
     if (ml[j].x == -INFINITY) continue;
-    add_state(ml[j].x, ml[j].y, v[j], M, sum, o);
+    add_state(ml[j].x, ml[j].y, v[j], M, t.c, sum, o);
   }
   if (GROUPS > 1) {
     if (dl == 0) {
@@ -758,7 +773,7 @@ __global__ __launch_bounds__(kTileThreads) void tree_attention_merge_kernel(cons
 #pragma unroll
     for (int w = 0; w < GROUPS; ++w) {
       if (sml[sub + w][0] == -INFINITY) continue;
-      add_state(sml[sub + w][0], sml[sub + w][1], sacc[sub + w][dl], M, sum, o);
+      add_state(sml[sub + w][0], sml[sub + w][1], sacc[sub + w][dl], M, t.c, sum, o);
     }
   }
   if (valid)
@@ -767,10 +782,12 @@ __global__ __launch_bounds__(kTileThreads) void tree_attention_merge_kernel(cons
 
 bool aligned(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
-// c = |scale| log2(e) must be a normal finite number: a masked score of -inf
-// times 0 would be NaN.
+// |scale| log2(e), the factor that takes scores to log2 units.  It must be a
+// normal finite number: a masked score of -inf times 0 would be NaN.
+float log2_scale(float scale) { return __builtin_fabsf(scale) * 1.44269504088896341f; }
+
 bool scale_ok(float scale) {
-  const float c = __builtin_fabsf(scale) * 1.44269504088896341f;
+  const float c = log2_scale(scale);
   return c >= 1.17549435e-38f && c <= 3.0e38f;
 }
 
@@ -843,6 +860,7 @@ int launch_tiled(const AttnArgs& a, int G, void* workspace, int64_t workspace_by
   t.row_tiles = p.row_tiles;
   t.splits = p.splits;
   t.split_keys = p.split_keys;
+  t.c = log2_scale(a.scale);
   if (p.splits > 1) {
     t.part_acc = static_cast<float*>(workspace);
     t.part_ml = reinterpret_cast<float2*>(

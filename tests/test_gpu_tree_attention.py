@@ -167,6 +167,44 @@ def test_fully_masked_row_is_zero_and_large_logits_are_stable(device):
     assert torch.isfinite(out.float()).all()
 
 
+# Scores past 2^24, where a rounded product of the row maximum is off by more
+# than the spacing of the exponents: both tile forms, masked and not, one and
+# many key splits.
+@pytest.mark.parametrize("std", [3e4, 1e5, 3e5, 1e15])
+@pytest.mark.parametrize("Q,S,masked", [(1, 4096, False), (61, 1085, True), (40, 100, True),
+                                        (200, 200, False), (1024, 1024, False),
+                                        (700, 900, True)])
+def test_large_finite_scores(device, Q, S, masked, std):
+    """At these scales one key takes all of a row's weight, so the row is that
+    key's values, bit for bit.  Rows whose two largest scores are closer than
+    the error of an fp32 dot product of 128 terms (2^-24 * 128 of the sum of
+    magnitudes, taken twice) are left out."""
+    Hq, Hkv, D, scale = 16, 2, 128, 128 ** -0.5
+    g = torch.Generator().manual_seed(Q + S)
+    q, k = _rand((Hq, Q, D), device, g, std), _rand((Hkv, S, D), device, g, std)
+    v = _rand((Hkv, S, D), device, g)
+    allowed = torch.arange(S, device=device)[None] <= S - Q + torch.arange(Q, device=device)[:, None]
+    mask = None
+    if masked:
+        allowed = (torch.rand((Q, S), generator=g) < 0.5).to(device)
+        allowed[:, 0] = True
+        mask = allowed[None, None].contiguous()
+    for sign in (1.0, -1.0):
+        out = ops.tree_attention(q[None], k[None], v[None], mask, sign * scale)[0]
+        decided = 0
+        for head in range(Hq):
+            kd = k[head * Hkv // Hq].double()
+            s = (sign * (q[head].double() @ kd.T)).masked_fill(~allowed, -math.inf)
+            size = (q[head].double().abs() @ kd.abs().T).amax(-1)
+            top = torch.cat([s, torch.full_like(s[:, :1], -math.inf)], dim=1).topk(2, dim=-1)
+            gap = top.values[:, 0] - top.values[:, 1]
+            rows = gap > 2 * 2 ** -24 * 128 * size + 200 / scale
+            decided += int(rows.sum())
+            want = v[head * Hkv // Hq][top.indices[:, 0]]
+            assert torch.equal(out[rows, head], want[rows]), (head, sign)
+        assert decided >= 0.9 * Q * Hq
+
+
 def test_argument_errors(device):
     q = torch.zeros((1, 4, 2, 8), dtype=torch.bfloat16, device=device)
     k = torch.zeros((1, 3, 5, 8), dtype=torch.bfloat16, device=device)
