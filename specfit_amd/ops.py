@@ -724,6 +724,10 @@ def tree_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
         return out
     if S == 0:
         return out.zero_()
+    if mask is not None:
+        if mask.shape[1] == 0:  # its address would be null: no mask, the causal rule
+            raise ValueError(f"mask must be bool [B, 1, {Q}, {S}]; it has no head")
+        mask_ptr = mask.data_ptr()
     lib = _native.lib()
     handle = _stream_handle(stream, device)
     # Scratch of a call whose keys are split over the chip; the calls of a
@@ -739,8 +743,6 @@ def tree_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     # shorter on the device than a handful of tensor operations on the host.
     (qb, qh, qt, _), (kb, kh, kt, _), (vb, vh, vt, _) = query.stride(), key.stride(), value.stride()
     q_ptr, k_ptr, v_ptr, out_ptr = query.data_ptr(), key.data_ptr(), value.data_ptr(), out.data_ptr()
-    if mask is not None:
-        mask_ptr = mask.data_ptr()
     for b in range(B):
         rc = lib.sf_tree_attention_split(
             q_ptr + 2 * b * qb, qt, qh, k_ptr + 2 * b * kb, kh, kt, v_ptr + 2 * b * vb, vh, vt,

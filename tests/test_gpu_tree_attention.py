@@ -205,6 +205,20 @@ def test_large_finite_scores(device, Q, S, masked, std):
         assert decided >= 0.9 * Q * Hq
 
 
+def test_mask_without_heads_is_refused(device):
+    """An empty head dimension holds no mask row; its null address must not
+    become the causal rule."""
+    q = torch.zeros((1, 4, 2, 64), dtype=torch.bfloat16, device=device)
+    k = torch.zeros((1, 2, 5, 64), dtype=torch.bfloat16, device=device)
+    for heads in (0, 4):
+        mask = torch.zeros((1, heads, 2, 5), dtype=torch.bool, device=device)
+        if heads:
+            assert not ops.tree_attention(q, k, k, mask, 1.0).any()  # head 0 serves every head
+        else:
+            with pytest.raises(ValueError, match="mask"):
+                ops.tree_attention(q, k, k, mask, 1.0)
+
+
 def test_argument_errors(device):
     q = torch.zeros((1, 4, 2, 8), dtype=torch.bfloat16, device=device)
     k = torch.zeros((1, 3, 5, 8), dtype=torch.bfloat16, device=device)
