@@ -697,7 +697,8 @@ def tree_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     unit last stride), mask [B, 1 or Hq, Q, S] bool (True = attend; the first
     head's mask is used) or None for causal attention aligned to the end of
     the keys.  Returns [B, Q, Hq, D] bf16, the layout HF attention functions
-    return."""
+    return.  With ``stream``, the inputs and the output (memory of the current
+    stream) are the caller's to order between the two streams."""
     for name, t in (("query", query), ("key", key), ("value", value)):
         _require_cuda(name, t, _BF16)
         if t.dim() != 4 or t.stride(-1) != 1:
@@ -731,14 +732,18 @@ def tree_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     lib = _native.lib()
     handle = _stream_handle(stream, device)
     # Scratch of a call whose keys are split over the chip; the calls of a
-    # batch run one after another on the stream and share it.
+    # batch run one after another on the stream and share it.  It comes from
+    # the pool of the stream that uses it: a block of another stream's pool
+    # may still be read there by kernels queued before it was given back.
     need = _attention_workspace(Q, S, Hq, Hkv, D, mask is not None)
     work_ptr = None
     if need:
-        work = torch.empty(need, dtype=torch.uint8, device=device)
+        if stream is None:
+            work = torch.empty(need, dtype=torch.uint8, device=device)
+        else:
+            with torch.cuda.stream(stream):
+                work = torch.empty(need, dtype=torch.uint8, device=device)
         work_ptr = work.data_ptr()
-        if stream is not None:  # may not be the stream the memory was allocated on
-            work.record_stream(stream)
     # Addresses and strides instead of per-batch views: this call is often
     # shorter on the device than a handful of tensor operations on the host.
     (qb, qh, qt, _), (kb, kh, kt, _), (vb, vh, vt, _) = query.stride(), key.stride(), value.stride()

@@ -248,6 +248,33 @@ def test_mask_without_heads_is_refused(device):
                 ops.tree_attention(q, k, k, mask, 1.0)
 
 
+def test_scratch_of_a_side_stream_call_is_the_side_streams(device):
+    """A block that the current stream gave back, with a copy from it still
+    queued there, is not the scratch of a call on another stream.  (The
+    output is the current stream's memory: nothing small is given back here
+    while it is in use.)"""
+    from specfit_amd import _native
+
+    g = torch.Generator().manual_seed(6)
+    q, k, v = (_rand((1, h, n, 128), device, g) for h, n in ((32, 1), (4, 4096), (4, 4096)))
+    ref = _reference(q, k, v, None, 0.09)
+    need = _native.lib().sf_tree_attention_workspace(1, 4096, 32, 4, 128, 0)
+    side, busy = torch.cuda.Stream(device), torch.randn(4096, 4096, device=device)
+    result = torch.empty_like(busy)
+    torch.cuda.synchronize()
+    block = torch.full((need,), 7, dtype=torch.uint8, device=device)
+    torch.cuda.synchronize()
+    for _ in range(20):  # several ms of work before the copy
+        torch.mm(busy, busy, out=result)
+    copy = block.clone()
+    del block
+    outs = [ops.tree_attention(q, k, v, None, 0.09, stream=side) for _ in range(3)]
+    torch.cuda.synchronize()
+    assert bool((copy == 7).all())
+    for out in outs:
+        _check(out, ref)
+
+
 def test_argument_errors(device):
     q = torch.zeros((1, 4, 2, 8), dtype=torch.bfloat16, device=device)
     k = torch.zeros((1, 3, 5, 8), dtype=torch.bfloat16, device=device)
