@@ -738,12 +738,15 @@ def tree_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
     need = _attention_workspace(Q, S, Hq, Hkv, D, mask is not None)
     work_ptr = None
     if need:
-        if stream is None:
-            work = torch.empty(need, dtype=torch.uint8, device=device)
-        else:
-            with torch.cuda.stream(stream):
+        try:
+            if stream is None:
                 work = torch.empty(need, dtype=torch.uint8, device=device)
-        work_ptr = work.data_ptr()
+            else:
+                with torch.cuda.stream(stream):
+                    work = torch.empty(need, dtype=torch.uint8, device=device)
+            work_ptr = work.data_ptr()
+        except torch.OutOfMemoryError:
+            need = 0  # the unsplit form needs no scratch
     # Addresses and strides instead of per-batch views: this call is often
     # shorter on the device than a handful of tensor operations on the host.
     (qb, qh, qt, _), (kb, kh, kt, _), (vb, vh, vt, _) = query.stride(), key.stride(), value.stride()

@@ -275,6 +275,25 @@ def test_scratch_of_a_side_stream_call_is_the_side_streams(device):
         _check(out, ref)
 
 
+def test_call_without_room_for_scratch_runs_unsplit(device, monkeypatch):
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (_rand((1, h, n, 128), device, g) for h, n in ((32, 1), (4, 4096), (4, 4096)))
+    ref = _reference(q, k, v, None, 0.09)
+    empty, refused = torch.empty, []
+
+    def full(*args, **kw):
+        if kw.get("dtype") is torch.uint8:
+            refused.append(args)
+            raise torch.OutOfMemoryError("no room")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", full)
+    out = ops.tree_attention(q, k, v, None, 0.09)
+    monkeypatch.undo()
+    assert refused
+    _check(out, ref)
+
+
 def test_argument_errors(device):
     q = torch.zeros((1, 4, 2, 8), dtype=torch.bfloat16, device=device)
     k = torch.zeros((1, 3, 5, 8), dtype=torch.bfloat16, device=device)
