@@ -329,10 +329,12 @@ int sf_tree_attention(const void *q, int64_t q_stride_token,
  * split its keys over the chip: each split's (max, sum, accumulator) goes to
  * the workspace in fp32 and a second kernel merges them in split order.
  * sf_tree_attention_workspace returns the bytes a call of that shape (masked:
- * with a mask) can use (0: it would not split).  workspace: device memory, 16-byte aligned, in use
- * until the call's kernels have run; with less than the needed bytes (or
- * NULL) the call runs unsplit.  Results of the two forms differ by the order
- * of the fp32 sums.
+ * with a mask) with 16-byte aligned rows can use (0: it would not split).
+ * workspace: device memory, 16-byte aligned, in use until the call's kernels
+ * have run; with less than the needed bytes (or NULL) the call runs unsplit.
+ * Results of the two forms differ by the order of the fp32 sums and by the
+ * rounding of probabilities to bf16, each relative to its form's running
+ * maximum.
  */
 int64_t sf_tree_attention_workspace(int queries, int keys, int q_heads,
                                     int kv_heads, int head_dim, int masked);

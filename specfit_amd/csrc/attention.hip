@@ -815,6 +815,13 @@ bool scale_ok(float scale) {
   return c >= 1.17549435e-38f && c <= 3.0e38f;
 }
 
+// Shapes of the tiled form: head dim 64 or 128, 2..16 query heads per KV head
+// (powers of two).
+bool tiled_shape(int queries, int G, int head_dim) {
+  return (head_dim == 64 || head_dim == 128) && G >= 2 && G <= 16 && (G & (G - 1)) == 0 &&
+         static_cast<int64_t>(queries) * G <= 0x3fffffff;
+}
+
 // Row groups (WR) and key splits of a call.
 struct TiledPlan {
   int wr, row_tiles, splits, split_keys;
@@ -993,14 +1000,12 @@ int attention_call(const void* q, int64_t q_stride_token, int64_t q_stride_head,
   a.scale = scale;
   a.out = static_cast<uint16_t*>(out);
   // The tiled form: 16-byte aligned query / key / value rows (8-element
-  // strides), head dim 64 or 128, 2..16 query heads per KV head, and a scale
-  // its log2 units can hold.
-  const bool tiled = aligned(q, 16) && aligned(v, 16) && aligned(out, 8) &&
-                     q_stride_token % 8 == 0 && q_stride_head % 8 == 0 &&
+  // strides) and a scale its log2 units can hold.
+  const bool tiled = tiled_shape(queries, G, head_dim) && aligned(q, 16) && aligned(v, 16) &&
+                     aligned(out, 8) && q_stride_token % 8 == 0 && q_stride_head % 8 == 0 &&
                      v_stride_token % 8 == 0 && v_stride_head % 8 == 0 &&
-                     k_stride_token < (1 << 24) && v_stride_token < (1 << 24) && G >= 2 &&
-                     G <= 16 && (G & (G - 1)) == 0 && scale_ok(scale) &&
-                     static_cast<int64_t>(queries) * G <= 0x3fffffff;
+                     k_stride_token < (1 << 24) && v_stride_token < (1 << 24) &&
+                     scale_ok(scale);
   if (tiled && head_dim == 128) return launch_tiled<128>(a, G, workspace, workspace_bytes, s);
   if (tiled && head_dim == 64) return launch_tiled<64>(a, G, workspace, workspace_bytes, s);
   switch (G) {
@@ -1031,9 +1036,7 @@ extern "C" int64_t sf_tree_attention_workspace(int queries, int keys, int q_head
                                                int head_dim, int masked) {
   if (queries < 1 || keys < 1 || kv_heads < 1 || q_heads < kv_heads || q_heads % kv_heads) return 0;
   const int G = q_heads / kv_heads;
-  if ((head_dim != 64 && head_dim != 128) || G > 16 ||
-      static_cast<int64_t>(queries) * G > 0x3fffffff)
-    return 0;
+  if (!tiled_shape(queries, G, head_dim)) return 0;
   return tiled_workspace(tiled_plan(queries, keys, kv_heads, G, masked != 0), queries, q_heads,
                          head_dim);
 }

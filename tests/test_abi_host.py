@@ -149,3 +149,14 @@ def test_workload_generator_is_seeded_and_zipf_skewed():
     h = make_hidden(4, 64, seed=1, zipf_fold=True)
     assert torch.all(h[:, 0] == 1.0)
     assert expected_distinct_uniform(16) == pytest.approx(82.4, abs=0.1)
+
+
+def test_attention_scratch_is_only_for_calls_that_split():
+    """Head dims, group sizes and sizes that the split form does not take have
+    no scratch: group sizes 1, 3 and 32 run unsplit or are refused."""
+    work = _native.lib().sf_tree_attention_workspace
+    for q_heads, kv_heads in [(32, 32), (12, 4), (24, 4), (64, 2)]:
+        for queries, keys, masked in [(1, 4096, 0), (61, 1085, 1), (129, 8129, 1)]:
+            assert work(queries, keys, q_heads, kv_heads, 128, masked) == 0, (q_heads, kv_heads)
+    for q_heads, kv_heads in [(8, 4), (16, 4), (32, 4), (64, 4)]:
+        assert work(1, 4096, q_heads, kv_heads, 128, 0) > 0
