@@ -831,15 +831,17 @@ struct TiledPlan {
 // 64-key tile at WR = 4, four at WR = 1) takes about 1.2 / 2.4 us on MI355X,
 // 1.6 / 2.9 us with a mask; splitting adds the merge launch (2.5 us on the
 // device, and 3 us of the caller's time with the scratch allocation, which
-// short calls wait for) and the partial states' way through memory (0.28 ns per row and split, 1 KiB each);
-// a CU runs one WR = 1 workgroup at a time, and WR = 4 workgroups above 1.5
-// per CU wait for each other.  Measured at 32 query / 4 KV heads of 128 (us):
-//   1 query, 4096 keys:     82.6 unsplit, 9.3 in 33 splits (WR = 4)
+// short calls wait for) and the partial states' way through memory (0.28 ns
+// per row and split, 1 KiB each); a CU runs one WR = 1 workgroup at a time,
+// and WR = 4 workgroups above 1.5 per CU wait for each other.  Measured at 32
+// query / 4 KV heads of 128 (us):
+//   1 query, 4097 keys:     82.6 unsplit, 9.0 in 33 splits (WR = 4); 43.7 unsplit (WR = 1)
 //   32 queries, 1056 keys:  21.8 unsplit, 12.2 in 5 (WR = 1); 13.4 WR = 4
 //   61 queries, 1085 keys:  22.0 unsplit, 15.9 in 3, 20.2 in 5 (WR = 1)
 //   129 queries, 8129 keys: 227 unsplit, 46.8 in 11, 54.3 in 32 (WR = 4)
 //   256 queries and keys:   8.8 unsplit (WR = 1), 10.9 (WR = 4), 13.9 in 2
-TiledPlan tiled_plan(int queries, int keys, int kv_heads, int G, bool mask) {
+// may_split: the caller has scratch for the partial states.
+TiledPlan tiled_plan(int queries, int keys, int kv_heads, int G, bool mask, bool may_split) {
   const int64_t rows = static_cast<int64_t>(queries) * G;
   TiledPlan best{};
   double best_cost = 0.0;
@@ -849,7 +851,7 @@ TiledPlan tiled_plan(int queries, int keys, int kv_heads, int G, bool mask) {
     const int64_t row_tiles = (rows + 32 * wr - 1) / (32 * wr);
     const int64_t blocks = row_tiles * kv_heads;
     const double step = wr == 4 ? (mask ? 1.6 : 1.2) : (mask ? 2.9 : 2.4);
-    const int most = units < kMaxSplits ? units : kMaxSplits;
+    const int most = !may_split ? 1 : units < kMaxSplits ? units : kMaxSplits;
     int last = 0;
     for (int want = 1; want <= most; ++want) {
       const int per = (units + want - 1) / want;
@@ -878,12 +880,13 @@ int64_t tiled_workspace(const TiledPlan& p, int queries, int q_heads, int head_d
 template <int D>
 int launch_tiled(const AttnArgs& a, int G, void* workspace, int64_t workspace_bytes,
                  hipStream_t s) {
-  TiledPlan p = tiled_plan(a.Q, a.S, a.Hkv, G, a.mask != nullptr);
+  // Without the scratch of the best split, the best unsplit form: its row
+  // groups may be others (one token over 4097 keys: 43.7 us, where the split
+  // plan's row groups in one split take 82.6).
+  TiledPlan p = tiled_plan(a.Q, a.S, a.Hkv, G, a.mask != nullptr, true);
   const int64_t need = tiled_workspace(p, a.Q, a.Hkv * G, D);
-  if (need > workspace_bytes || (need && (!workspace || !aligned(workspace, 16)))) {
-    p.splits = 1;
-    p.split_keys = a.S;
-  }
+  if (need > workspace_bytes || (need && (!workspace || !aligned(workspace, 16))))
+    p = tiled_plan(a.Q, a.S, a.Hkv, G, a.mask != nullptr, false);
   TiledArgs t{};
   t.a = a;
   t.log_g = __builtin_ctz(G);
@@ -1037,8 +1040,8 @@ extern "C" int64_t sf_tree_attention_workspace(int queries, int keys, int q_head
   if (queries < 1 || keys < 1 || kv_heads < 1 || q_heads < kv_heads || q_heads % kv_heads) return 0;
   const int G = q_heads / kv_heads;
   if (!tiled_shape(queries, G, head_dim)) return 0;
-  return tiled_workspace(tiled_plan(queries, keys, kv_heads, G, masked != 0), queries, q_heads,
-                         head_dim);
+  return tiled_workspace(tiled_plan(queries, keys, kv_heads, G, masked != 0, true), queries,
+                         q_heads, head_dim);
 }
 
 extern "C" int sf_tree_attention_split(const void* q, int64_t q_stride_token,

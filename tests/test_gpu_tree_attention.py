@@ -294,6 +294,37 @@ def test_call_without_room_for_scratch_runs_unsplit(device, monkeypatch):
     _check(out, ref)
 
 
+def test_call_without_scratch_uses_the_best_unsplit_form(device):
+    """One token over 4096 keys without scratch: four key groups in a
+    workgroup, about 5 times the split call's device time (9 us); one key
+    group takes 9 times."""
+    from specfit_amd import _native
+
+    lib, stream = _native.lib(), torch.cuda.current_stream(device).cuda_stream
+    Hq, Hkv, D, S = 32, 4, 128, 4096
+    q, k, v, out = (torch.randn(s, device=device).to(torch.bfloat16)
+                    for s in ((1, Hq, D), (Hkv, S, D), (Hkv, S, D), (1, Hq, D)))
+    need = lib.sf_tree_attention_workspace(1, S, Hq, Hkv, D, 0)
+    work = torch.empty(need, dtype=torch.uint8, device=device)
+
+    def seconds(work_ptr, nbytes):
+        times = []
+        for _ in range(7):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(50):
+                _native.check(lib.sf_tree_attention_split(
+                    q.data_ptr(), Hq * D, D, k.data_ptr(), S * D, D, v.data_ptr(), S * D, D, None,
+                    0, 1, S, Hq, Hkv, D, 0.09, out.data_ptr(), work_ptr, nbytes, stream), "split")
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return sorted(times)[3]
+
+    split, whole = seconds(work.data_ptr(), need), seconds(None, 0)
+    assert whole < 7 * split, (whole, split)
+
+
 def test_argument_errors(device):
     q = torch.zeros((1, 4, 2, 8), dtype=torch.bfloat16, device=device)
     k = torch.zeros((1, 3, 5, 8), dtype=torch.bfloat16, device=device)
