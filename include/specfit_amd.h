@@ -198,6 +198,23 @@ int sf_grouped_swiglu_table(const void *hidden, const int32_t *perm_pos,
                             sf_stream_t stream);
 
 /*
+ * sf_grouped_swiglu_table with a bound on the number of slot_of_expert's
+ * entries that are not -1 (0: not known), which picks between the kernels for
+ * few and for many rows.  The results do not depend on it.
+ */
+int sf_grouped_swiglu_table_residents(const void *hidden, const int32_t *perm_pos,
+                                      const int32_t *offsets,
+                                      const void *route_weights, int tokens,
+                                      int top_k, int hidden_size,
+                                      int intermediate_size, int num_experts,
+                                      int max_rows, int residents,
+                                      const int32_t *slot_of_expert,
+                                      const void *slot_base,
+                                      int64_t slot_stride_elems,
+                                      void *act_workspace, void *out_rows,
+                                      sf_stream_t stream);
+
+/*
  * K3, device slot-table form, allocating nothing.  No counterpart in the
  * reference: this entry point is for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that

@@ -30,6 +30,8 @@ SIGNATURES = {
     "sf_grouped_swiglu": ([_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p],
                           _i),
     "sf_grouped_swiglu_table": ([_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _i64, _p, _p, _p], _i),
+    "sf_grouped_swiglu_table_residents": ([_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _i64,
+                                           _p, _p, _p], _i),
     "sf_grouped_swiglu_table_noalloc": ([_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _i64, _p,
                                          _p], _i),
     "sf_expert_swiglu": ([_p, _i, _i64, _i, _i, _p, _p, _p, _p], _i),

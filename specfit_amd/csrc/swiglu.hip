@@ -1054,32 +1054,63 @@ int launch_width(const SwigluArgs& a, int groups, int max_rows, hipStream_t s) {
   return launch_class<R, 2, NBG, NBD>(a, groups, max_rows, s);
 }
 
-// The many-row kernels run where an expert may need a second pass of the
-// streaming split (above 128 rows), and for 65..128 rows where the launch has
-// enough of their larger tiles: from 8 experts at I = 768, 4 at I = 1536 (a
-// launch that leaves most CUs without a tile waits for one workgroup's whole
-// k loop, ~42 us).  Streaming / many-row, us, (H, I) = (2048, 768), experts
-// of 100 rows: 4: 29 / 47, 8: 49 / 48, 12: 68 / 58, 24: 116 / 82, 48: 209 /
-// 140; of 400 rows: 1: 85 / 45, 8: 159 / 73, 48: 751 / 332; (4096, 1536), 100
-// rows: 2: 47 / 81, 4: 86 / 84, 8: 138 / 93, 32: 525 / 272.  Slot-table
-// launches (T bounds the rows; most experts have fewer) at 128 experts,
-// uniform routing: T = 65: 244 / 214, 256: 272 / 232, 1024: 425 / 287, 2048:
-// 751 / 365; Zipf: T = 100: 118 / 120, 256: 209 / 169, 2048: 975 / 469.
-// A slot-table launch of few experts with up to 32 rows on average streams:
-// 32 experts of (4096, 1536), T = 100: 263 / 268, 128: 268 / 280.
-bool wide_launch(const SwigluArgs& a, Resolve r, int groups, int max_rows, long long tokens) {
+// Where the many-row kernels run: where the launch has enough of their larger
+// tiles to fill the chip (one that leaves most CUs without a tile waits for
+// one workgroup's whole k loop, 35 - 50 us at I = 768, twice that at 1536), or
+// an expert needs so many passes of the streaming split that they take longer.
+// All figures: streaming / many-row, us.
+//
+// Rows known on the host (lists, one expert): 8 streaming passes of experts
+// above 64 rows at I = 768, 4 at 1536, or an expert of more than 224 rows.
+// (H, I) = (2048, 768), n experts of 100 rows: 4: 28 / 48, 8: 48 / 49, 12: 68 /
+// 58, 48: 209 / 140; of 70: 8: 40 / 42, 12: 57 / 47; one of 100 and 7 of 20: 34 /
+// 53; 4 of 100 and 20 of 30: 63 / 67; one expert of 129: 36 / 49, 200: 44 / 43,
+// 256: 50 / 43, 400: 82 / 50; 140 and 11 of 20: 47 / 61; 400 and 11 of 5: 91 / 61.
+// (4096, 1536): 4 of 100: 86 / 86, 8: 137 / 92; 128, 100, 80 and five below 65:
+// 99 / 100; 200 and 7 of 20: 93 / 105; 300, 200, 100 and five below 65: 135 / 143.
+//
+// Slot tables: the rows are on the device only; `residents` bounds the table's
+// entries that are not -1 (0: unknown, then all may be).  With most experts
+// resident: every launch of more than 64 tokens at 128 experts (uniform
+// routing: T = 65: 217 / 202, 256: 247 / 220, 2048: 737 / 327; Zipf: 96: 121 /
+// 120, 256: 194 / 155, 2048: 837 / 407), and above 32 rows on average at few
+// experts (32 of (4096, 1536): T = 128: 261 / 263, 160: 278 / 248, 512: 723 /
+// 306).  With few, from 1536 expected rows (I = 768) on; below, a few popular
+// experts leave the chip idle in the tiled form (Zipf routing, the most popular
+// resident: 12 slots: T = 65: 41 / 56, 128: 69 / 74; 24 slots: 61 / 66, 89 / 84)
+// and so do few experts of 33..64 rows (uniform: 12 slots: T = 512: 43 / 50,
+// 2048: 90 / 84; 24 slots: 512: 69 / 81, 1024: 96 / 84; 8 slots: 2048: 67 / 81).
+// That gives up the popular ones' gain between (12 slots, T = 512: 193 / 94).
+bool wide_launch(const SwigluArgs& a, Resolve r, int groups, int max_rows, long long tokens,
+                 int residents) {
   if (max_rows <= 64 || tokens * a.row_stride >= (1ll << 31)) return false;  // 32-bit byte offsets
-  if (r == Resolve::kTable && groups < 64 && tokens * a.top_k <= 32ll * groups) return false;
-  return max_rows > 128 || groups * static_cast<long long>(a.I) >= 8 * 768;
+  if (r == Resolve::kDense || a.rows_known) {
+    long long passes = 0;
+    int most = 0;
+    for (int i = 0; i < groups; ++i) {
+      const int m = r == Resolve::kDense ? a.dense_m : a.rows[i];
+      if (m > 64) passes += (m + 127) / 128;
+      if (m > most) most = m;
+    }
+    return most > 224 || passes * a.I >= 8 * 768;
+  }
+  if (tokens <= 64) return false;  // rows of one expert, unless a token names it twice
+  const long long routes = tokens * a.top_k;
+  if (r == Resolve::kTable && 4ll * residents >= 3ll * groups) {
+    if (groups < 64 && routes <= 32ll * groups) return false;
+    return max_rows > 128 || groups * static_cast<long long>(a.I) >= 8 * 768;
+  }
+  const long long rows = r == Resolve::kTable && residents > 0 ? routes * residents / groups : routes;
+  return rows * a.I >= 1536 * 768;
 }
 
 // max_rows bounds the rows of any expert of the launch; it picks the row
-// class of the build.  tokens: rows of a.hidden.
+// class of the build.  tokens: rows of a.hidden.  residents: see wide_launch.
 template <Resolve R>
 int launch(const SwigluArgs& a, int groups, Shape shape, int max_rows, long long tokens,
-           hipStream_t s) {
+           int residents, hipStream_t s) {
   if (groups <= 0) return SF_OK;
-  if (wide_launch(a, R, groups, max_rows, tokens)) {
+  if (wide_launch(a, R, groups, max_rows, tokens, residents)) {
     if (shape == Shape::k2048x768) return launch_wide<R, 8, 3>(a, groups, s);
     if (shape == Shape::k4096x1536) return launch_wide<R, 16, 6>(a, groups, s);
   }
@@ -1154,7 +1185,7 @@ extern "C" int sf_grouped_swiglu(const void* hidden, const int32_t* perm_pos,
         a.rows[i] = expert_row_count[base + i];
       }
     }
-    rc = launch<Resolve::kList>(a, a.n, shape, max_rows, tokens, s);
+    rc = launch<Resolve::kList>(a, a.n, shape, max_rows, tokens, 0, s);
     if (rc) return rc;
   }
   return SF_OK;
@@ -1162,11 +1193,12 @@ extern "C" int sf_grouped_swiglu(const void* hidden, const int32_t* perm_pos,
 
 namespace {
 
-// Slot-table launch shared by sf_grouped_swiglu_table and its
-// allocation-free variant; `act` is the activation workspace.
+// Slot-table launch shared by sf_grouped_swiglu_table, its form with the
+// resident count and its allocation-free variant; `act` is the activation
+// workspace, residents 0 where the caller does not say.
 int table_launch(const void* hidden, const int32_t* perm_pos, const int32_t* offsets,
                  const void* route_weights, int tokens, int top_k, int hidden_size,
-                 int intermediate_size, int num_experts, int max_rows,
+                 int intermediate_size, int num_experts, int max_rows, int residents,
                  const int32_t* slot_of_expert, const void* slot_base,
                  int64_t slot_stride_elems, void* act, void* out_rows, hipStream_t stream) {
   const bool aligned = aligned16(hidden) && aligned16(act) && aligned16(slot_base) &&
@@ -1187,7 +1219,7 @@ int table_launch(const void* hidden, const int32_t* perm_pos, const int32_t* off
   a.slot_of_expert = slot_of_expert;
   a.slot_base = static_cast<const uint16_t*>(slot_base);
   a.slot_stride = slot_stride_elems;
-  return launch<Resolve::kTable>(a, num_experts, shape, max_rows, tokens, stream);
+  return launch<Resolve::kTable>(a, num_experts, shape, max_rows, tokens, residents, stream);
 }
 
 int check_table(int tokens, int top_k, int hidden_size, int intermediate_size, int num_experts,
@@ -1246,6 +1278,25 @@ int scratch_address(hipStream_t stream, void** out) {
 
 }  // namespace
 
+extern "C" int sf_grouped_swiglu_table_residents(
+    const void* hidden, const int32_t* perm_pos, const int32_t* offsets, const void* route_weights,
+    int tokens, int top_k, int hidden_size, int intermediate_size, int num_experts, int max_rows,
+    int residents, const int32_t* slot_of_expert, const void* slot_base, int64_t slot_stride_elems,
+    void* act_workspace, void* out_rows, sf_stream_t stream) {
+  const int rc = check_table(tokens, top_k, hidden_size, intermediate_size, num_experts,
+                             max_rows, slot_stride_elems);
+  if (rc) return rc;
+  if (residents < 0) return SF_ERR_INVALID_ARGUMENT;
+  if (tokens == 0) return SF_OK;
+  if (!hidden || !perm_pos || !offsets || !slot_of_expert || !slot_base ||
+      !act_workspace || !out_rows)
+    return SF_ERR_INVALID_ARGUMENT;
+  return table_launch(hidden, perm_pos, offsets, route_weights, tokens, top_k, hidden_size,
+                      intermediate_size, num_experts, max_rows, residents, slot_of_expert,
+                      slot_base, slot_stride_elems, act_workspace, out_rows,
+                      reinterpret_cast<hipStream_t>(stream));
+}
+
 extern "C" int sf_grouped_swiglu_table(const void* hidden, const int32_t* perm_pos,
                                        const int32_t* offsets, const void* route_weights,
                                        int tokens, int top_k, int hidden_size,
@@ -1254,17 +1305,10 @@ extern "C" int sf_grouped_swiglu_table(const void* hidden, const int32_t* perm_p
                                        const void* slot_base, int64_t slot_stride_elems,
                                        void* act_workspace, void* out_rows,
                                        sf_stream_t stream) {
-  const int rc = check_table(tokens, top_k, hidden_size, intermediate_size, num_experts,
-                             max_rows, slot_stride_elems);
-  if (rc) return rc;
-  if (tokens == 0) return SF_OK;
-  if (!hidden || !perm_pos || !offsets || !slot_of_expert || !slot_base ||
-      !act_workspace || !out_rows)
-    return SF_ERR_INVALID_ARGUMENT;
-  return table_launch(hidden, perm_pos, offsets, route_weights, tokens, top_k, hidden_size,
-                      intermediate_size, num_experts, max_rows, slot_of_expert, slot_base,
-                      slot_stride_elems, act_workspace, out_rows,
-                      reinterpret_cast<hipStream_t>(stream));
+  return sf_grouped_swiglu_table_residents(
+      hidden, perm_pos, offsets, route_weights, tokens, top_k, hidden_size, intermediate_size,
+      num_experts, max_rows, 0, slot_of_expert, slot_base, slot_stride_elems, act_workspace,
+      out_rows, stream);
 }
 
 extern "C" int sf_grouped_swiglu_table_noalloc(const void* hidden, const int32_t* perm_pos,
@@ -1288,7 +1332,7 @@ extern "C" int sf_grouped_swiglu_table_noalloc(const void* hidden, const int32_t
   const int sr = scratch_address(s, &act);
   if (sr) return sr;
   return table_launch(hidden, perm_pos, offsets, route_weights, tokens, top_k, hidden_size,
-                      intermediate_size, num_experts, max_rows, slot_of_expert, slot_base,
+                      intermediate_size, num_experts, max_rows, 0, slot_of_expert, slot_base,
                       slot_stride_elems, act, out_rows, s);
 }
 
@@ -1314,5 +1358,5 @@ extern "C" int sf_expert_swiglu(const void* rows, int m, int64_t row_stride,
   a.dense_m = m;
   a.n = 1;
   a.wptr[0] = reinterpret_cast<uint64_t>(packed_weights);
-  return launch<Resolve::kDense>(a, 1, shape, m, m, reinterpret_cast<hipStream_t>(stream));
+  return launch<Resolve::kDense>(a, 1, shape, m, m, 0, reinterpret_cast<hipStream_t>(stream));
 }

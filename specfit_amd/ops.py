@@ -513,11 +513,13 @@ def grouped_swiglu_table(hidden: torch.Tensor, plan: DispatchPlan,
                          slot_storage: torch.Tensor, hidden_size: int, intermediate_size: int,
                          act: torch.Tensor, out_rows: torch.Tensor, *,
                          max_rows: int | None = None, stream: torch.cuda.Stream | None = None,
-                         tag: str = "") -> list | None:
+                         tag: str = "", residents: int | None = None) -> list | None:
     """K3 over every expert whose device slot-table entry is >= 0 (no host
     knowledge of the active set needed).  ``max_rows`` bounds any expert's
     rows (default tokens * top_k; tokens when every token's experts are
-    distinct).  While launches are recorded, returns the recorder's entry
+    distinct).  ``residents`` bounds the number of table entries >= 0 (default:
+    the rows of ``slot_storage``); it picks kernels and changes no result.
+    While launches are recorded, returns the recorder's entry
     ``[experts, rows, tag, start, end]``: the caller fills in the first two
     once it knows which experts had rows."""
     if plan.tokens == 0:
@@ -534,17 +536,19 @@ def grouped_swiglu_table(hidden: torch.Tensor, plan: DispatchPlan,
     bound = N if max_rows is None else int(max_rows)
     if bound < 1:
         raise ValueError("max_rows must be positive")
+    if residents is None:
+        residents = slot_storage.shape[0]
     rec = _recorder
     entry = None
     if rec is not None:
         s = stream if stream is not None else torch.cuda.current_stream(hidden.device)
         start, end = rec._events(s)
-    rc = _native.lib().sf_grouped_swiglu_table(
+    rc = _native.lib().sf_grouped_swiglu_table_residents(
         _ptr(hidden), _ptr(plan.perm_pos), _ptr(plan.offsets), _ptr(route_weights),
         plan.tokens, plan.top_k, hidden_size, intermediate_size, plan.num_experts, bound,
-        _ptr(slot_of_expert), _ptr(slot_storage), int(slot_storage.stride(0)),
+        int(residents), _ptr(slot_of_expert), _ptr(slot_storage), int(slot_storage.stride(0)),
         _ptr(act), _ptr(out_rows), _stream_handle(stream, hidden.device))
-    _native.check(rc, "sf_grouped_swiglu_table")
+    _native.check(rc, "sf_grouped_swiglu_table_residents")
     if rec is not None:
         end.record(s)
         entry = [0, 0, tag, start, end]

@@ -245,7 +245,8 @@ class Qwen3OffloadedExperts(nn.Module):
             entry = ops.grouped_swiglu_table(routes.hidden, plan, routes.route_weights, table,
                                              routes.storage, self.hidden_size,
                                              self.intermediate_size, routes.act, routes.rows,
-                                             max_rows=T, tag="resident")
+                                             max_rows=T, tag="resident",
+                                             residents=num_experts - slots.count(-1) if T > 64 else None)
             counts = self._read_counts(plan, top_k_index, num_experts)
             active = tuple(compress(range(num_experts), counts))
             routes.covered = frozenset(e for e in active if slots[e] >= 0 and counts[e] <= T)

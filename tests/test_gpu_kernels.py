@@ -395,6 +395,62 @@ def test_many_row_kernels_match_the_streaming_split(device, H, I):
         assert torch.equal(y[lo:lo + 128], ops.expert_swiglu(x[lo:lo + 128], slots[2], H, I))
 
 
+def _device_us(launch, calls=10):
+    """Device time of one launch: the median of 7 replays of a captured run."""
+    launch()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(calls):
+            launch()
+    times = []
+    for _ in range(7):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        graph.replay()
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end) * 1e3 / calls)
+    return sorted(times)[3]
+
+
+def test_few_large_experts_stream(device):
+    """Launches with a few experts above 64 rows leave the chip idle in the
+    tiled kernels (50 us at this shape for one expert's k loop): they take the
+    streaming ones.  The bars are half way between the two on either side."""
+    H, I, E = 2048, 768, 8
+    g = torch.Generator("cpu").manual_seed(3)
+    slots = (torch.randn(E, 3 * H * I, generator=g) * 0.03).to(torch.bfloat16).to(device)
+
+    def case(counts, T):
+        idx = torch.full((T, E), -1, dtype=torch.int64)
+        for e, m in enumerate(counts):
+            idx[:m, e] = e
+        plan = ops.dispatch(idx.to(device), E)
+        plan.fetch_counts()
+        hidden = torch.randn(T, H, generator=g).to(torch.bfloat16).to(device)
+        act = torch.empty((T * E, I), dtype=torch.bfloat16, device=device)
+        return hidden, plan, act, torch.empty((T * E, H), dtype=torch.bfloat16, device=device)
+
+    def listed(counts, T):
+        hidden, plan, act, rows = case(counts, T)
+        return _device_us(lambda: ops.grouped_swiglu(
+            hidden, plan, None, range(E), list(slots), H, I, act, rows, slot_storage=slots))
+
+    even = listed([100] * E, 128)  # 8 experts of 100 rows: either form takes 48 us
+    skewed = listed([100] + [20] * (E - 1), 128)
+    assert skewed < 0.9 * even, (skewed, even)  # 34 streaming, 53 tiled
+    hidden, plan, act, rows = case([100] * E, 128)
+    x = hidden[:1].expand(129, H).contiguous()
+    one, more = (_device_us(lambda n=n: ops.expert_swiglu(x[:n], slots[0], H, I)) for n in (128, 129))
+    assert more < 1.6 * one, (more, one)  # 36 streaming, 49 tiled, against 27
+    # A table with 2 of the 8 experts resident, popular ones.
+    table = torch.tensor([0, 1] + [-1] * (E - 2), dtype=torch.int32, device=device)
+    few = _device_us(lambda: ops.grouped_swiglu_table(
+        hidden, plan, None, table, slots[:2], H, I, act, rows, max_rows=128))
+    assert few < 1.4 * one, (few, one)  # 28 streaming, 45 tiled
+
+
 @pytest.mark.parametrize("H,I,m", [(4, 3, 2), (32, 16, 5), (96, 64, 70), (2048, 768, 48),
                                    (2048, 768, 130), (4096, 1536, 20), (4096, 1536, 70)])
 def test_expert_swiglu_generic_and_mfma_paths(device, H, I, m):
