@@ -1084,6 +1084,7 @@ int launch_width(const SwigluArgs& a, int groups, int max_rows, hipStream_t s) {
 bool wide_launch(const SwigluArgs& a, Resolve r, int groups, int max_rows, long long tokens,
                  int residents) {
   if (max_rows <= 64 || tokens * a.row_stride >= (1ll << 31)) return false;  // 32-bit byte offsets
+  if (reinterpret_cast<uintptr_t>(a.out) % 8) return false;  // 8-byte stores
   if (r == Resolve::kDense || a.rows_known) {
     long long passes = 0;
     int most = 0;

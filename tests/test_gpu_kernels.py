@@ -395,6 +395,26 @@ def test_many_row_kernels_match_the_streaming_split(device, H, I):
         assert torch.equal(y[lo:lo + 128], ops.expert_swiglu(x[lo:lo + 128], slots[2], H, I))
 
 
+def test_many_rows_into_unaligned_output_rows(device):
+    """The tiled kernels store 8 bytes at a time; output rows off that
+    alignment take the streaming kernels, with the same bits."""
+    H, I, E, T = 2048, 768, 2, 300
+    g = torch.Generator("cpu").manual_seed(8)
+    hidden = torch.randn(T, H, generator=g).to(torch.bfloat16).to(device)
+    slots = (torch.randn(E, 3 * H * I, generator=g) * 0.03).to(torch.bfloat16).to(device)
+    plan = ops.dispatch(torch.arange(E, device=device).expand(T, E).contiguous(), E)
+    table = torch.arange(E, dtype=torch.int32, device=device)
+    act = torch.empty((T * E, I), dtype=torch.bfloat16, device=device)
+    want = torch.empty((T * E, H), dtype=torch.bfloat16, device=device)
+    ops.grouped_swiglu_table(hidden, plan, None, table, slots, H, I, act, want, max_rows=T)
+    for shift in (1, 2, 3, 4):
+        buf = torch.zeros(T * E * H + 8, dtype=torch.bfloat16, device=device)
+        rows = buf[shift:shift + T * E * H].view(T * E, H)
+        ops.grouped_swiglu_table(hidden, plan, None, table, slots, H, I, act, rows, max_rows=T)
+        assert torch.equal(rows, want), shift
+        assert not buf[:shift].any() and not buf[shift + T * E * H:].any()
+
+
 def _device_us(launch, calls=10):
     """Device time of one launch: the median of 7 replays of a captured run."""
     launch()
