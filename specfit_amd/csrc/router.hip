@@ -199,12 +199,17 @@ __global__ __launch_bounds__(kLogitWaves * SF_WAVE) void router_logits_kernel(
 // bits are the same.  Bound by the vector ALU (2048 of its 2754 instructions
 // per tile are the multiply-adds of H = 2048).  Any H of whole chunk rounds
 // (512 elements).
-// Taken from 32768 logits on, where its tiles fill the chip: both kernels of
-// the call at E = 128, small / large tile, us: H = 2048, T = 128: 9.5 / 12.4,
-// 256: 13.0 / 12.6, 512: 20.1 / 12.9, 2048: 57.5 / 26.6; H = 4096, T = 192:
-// 15.5 / 18.8, 256: 18.5 / 19.2, 384: 24.5 / 19.5, 2048: 101 / 42.7.
+// Taken where its tiles fill the chip, from 40960 logits on up to H = 4096 and
+// from 32768 above.  Both kernels of the call, small / large tile, us: E = 128,
+// H = 1024, T = 256: 9.2 / 9.7, 384: 10.7 / 9.8, 2048: 26.2 / 16.7; H = 2048, T =
+// 256: 13.1 / 12.9, 512: 19.6 / 13.1, 2048: 53.3 / 24.4; H = 4096, T = 256: 19.1
+// / 19.1, 384: 25.5 / 19.4, 2048: 94.9 / 40.6; H = 6144, T = 256: 33.8 / 25.2.
+// E = 256, T = 128: H = 1024: 10.8 / 11.3, 4096: 19.9 / 20.4, 8192: 40.7 / 36.3;
+// E = 8 (three of a workgroup's four wavefronts idle), T = 4096: H = 1024: 9.8 /
+// 9.9, 4096: 21.2 / 20.7, T = 16384: 24.3 / 20.6, 64.6 / 44.4.
 constexpr int kManyTile = 8;  // tokens and experts of a wavefront
-constexpr long long kManyLogits = 32768;
+
+long long many_logits(int hidden_size) { return hidden_size <= 4096 ? 40960 : 32768; }
 
 template <int CTRL>
 __device__ __forceinline__ float butterfly_pair(float even, float odd, bool bit) {
@@ -374,7 +379,7 @@ extern "C" int sf_router_topk(const void* hidden, const void* router_weight,
   const int nchunks = (hidden_size + 7) / 8;
   const int per_lane = (nchunks + SF_WAVE - 1) / SF_WAVE;
   const bool many = aligned && hidden_size % (8 * SF_WAVE) == 0 &&
-                    static_cast<long long>(tokens) * num_experts >= kManyLogits &&
+                    static_cast<long long>(tokens) * num_experts >= many_logits(hidden_size) &&
                     static_cast<long long>(tokens) * hidden_size < (1ll << 31) &&
                     static_cast<long long>(num_experts) * hidden_size < (1ll << 31);
   if (aligned && (many || per_lane <= 16)) {

@@ -78,6 +78,13 @@ def test_router_bitexact_many_tokens(device, T, H, E, K):
     _router_case(device, T, H, E, K, True, 33)
 
 
+# Either side of the line between the tiles, for both of its values.
+@pytest.mark.parametrize("T,H,E", [(319, 2048, 128), (320, 2048, 128), (160, 4096, 256),
+                                   (255, 4608, 128), (256, 4608, 128), (5120, 512, 8)])
+def test_router_bitexact_at_the_tile_line(device, T, H, E):
+    _router_case(device, T, H, E, 8, True, 34)
+
+
 def test_router_ties_resolve_to_lower_id(device):
     h = torch.zeros(3, 256, dtype=torch.bfloat16)
     w = _randn_bf16((16, 256), 4, 0.02)
