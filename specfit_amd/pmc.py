@@ -73,6 +73,12 @@ def _is_table(name: str) -> bool:
     return bool(m) and m.group(1) == "1"
 
 
+def _is_many_row(name: str) -> bool:
+    """A many-row K3 dispatch.  Its grid is padded to groups of 8 experts, so
+    it does not give the number of experts nor their weight bytes."""
+    return "gateup_wide_kernel" in name or "down_wide_kernel" in name
+
+
 def _k3_weight_bytes(name: str, grid: int) -> int | None:
     if "gateup_mfma_kernel" in name:
         cols = 8 * _tile_width(name)
@@ -142,6 +148,10 @@ def summarize(fetch_dir: str, write_dir: str, command: str | None = None) -> str
             lines.append(f"| {label} | {pairs} | {key} | {n} | {fb / n / 1e6:.2f} | "
                          f"{wb / n / 1e6:.3f} | {ab / n / 1e6:.2f} | {fb / ab:.3f} |")
         ratios[label] = ((fetch + write) / alg, fetch / pairs, write / pairs, alg / pairs)
+    many = sum(_is_many_row(d[1]) for d in f_disp)
+    if many:
+        lines += ["", f"{many} dispatches of the many-row K3 kernels are in none of these rows: "
+                  "their grid does not give their experts."]
     # Coded-transfer decodes (sf_expert_decode) before the calibration kernel.
     f_cal = [i for i, d in enumerate(f_disp) if CALIBRATION_TAG in d[1]][0]
     w_cal = [i for i, d in enumerate(w_disp) if CALIBRATION_TAG in d[1]][0]
@@ -170,14 +180,16 @@ def summarize(fetch_dir: str, write_dir: str, command: str | None = None) -> str
 
 
 # Kernel names of libspecfit_amd (K1-K8), listed in the trace summaries.
-LIBRARY_KERNELS = ("router_logits_kernel", "router_select_kernel", "dispatch_kernel",
-                   "gateup_mfma_kernel", "down_mfma_kernel", "gateup_generic_kernel",
+LIBRARY_KERNELS = ("router_logits_kernel", "router_logits_many_kernel", "router_select_kernel",
+                   "dispatch_kernel", "gateup_mfma_kernel", "down_mfma_kernel",
+                   "gateup_wide_kernel", "down_wide_kernel", "gateup_generic_kernel",
                    "down_generic_kernel", "combine_kernel", "decode_kernel",
                    "tree_attention_kernel", "tree_attention_tiled_kernel",
-                   "tree_attention_merge_kernel", "rms_norm_kernel", "qk_norm_rope_kernel", "router_topk_scalar_kernel")
+                   "tree_attention_merge_kernel", "rms_norm_kernel", "qk_norm_rope_kernel",
+                   "router_topk_scalar_kernel")
 
 
-FORWARD_START = "router_logits_kernel"
+FORWARD_START = "router_logits_"  # of few or of many tokens
 
 
 def _stats_of(trace: list[dict]) -> list[dict]:
@@ -247,7 +259,8 @@ def summarize_trace(trace_dir: str, command: str | None = None,
                          f"{float(r['Percentage']):.1f}% |")
     cal = [i for i, r in enumerate(trace) if CALIBRATION_TAG in r["Kernel_Name"]]
     k3 = [(i, r) for i, r in enumerate(trace)
-          if "gateup_mfma_kernel" in r["Kernel_Name"] or "down_mfma_kernel" in r["Kernel_Name"]]
+          if "gateup_mfma_kernel" in r["Kernel_Name"] or "down_mfma_kernel" in r["Kernel_Name"]
+          or _is_many_row(r["Kernel_Name"])]
     lines += ["", "## K3 launches (gate/up + down dispatch pairs)", "",
               "| phase | launches | avg gate/up µs | avg down µs | avg launch µs (sum) | "
               "avg weight MB | GB/s (weights / kernel time) |", "|---|---|---|---|---|---|---|"]
@@ -256,15 +269,17 @@ def summarize_trace(trace_dir: str, command: str | None = None,
               else (("all", [r for _, r in k3]),))
     dur = lambda rs: sum(int(r["End_Timestamp"]) - int(r["Start_Timestamp"]) for r in rs) / len(rs) / 1e3
     for label, sel in phases:
-        for table in (False, True):
-            part = [r for r in sel if _is_table(r["Kernel_Name"]) == table]
+        for table, many in ((False, False), (True, False), (False, True), (True, True)):
+            part = [r for r in sel if _is_table(r["Kernel_Name"]) == table
+                    and _is_many_row(r["Kernel_Name"]) == many]
             g = [r for r in part if "gateup" in r["Kernel_Name"]]
-            d = [r for r in part if "down_mfma" in r["Kernel_Name"]]
+            d = [r for r in part if "down" in r["Kernel_Name"]]
             if not g or len(g) != len(d):
                 continue
             t = dur(g) + dur(d)
-            if table:  # the grid covers every table entry, not the experts computed
-                lines.append(f"| {label}, slot table | {len(g)} | {dur(g):.2f} | {dur(d):.2f} | "
+            if table or many:  # the grid covers more than the experts computed
+                name = label + (", slot table" if table else "") + (", many rows" if many else "")
+                lines.append(f"| {name} | {len(g)} | {dur(g):.2f} | {dur(d):.2f} | "
                              f"{t:.2f} | n/a | n/a |")
                 continue
             wb = sum(_k3_weight_bytes(r["Kernel_Name"], int(r["Grid_Size_X"])) for r in part) / len(g)

@@ -180,6 +180,61 @@ def test_trace_summary_without_split_starts_at_the_first_router(tmp_path):
     assert "| `router_logits_kernel<4>` | 2 | 5.00 | 4.00 | 6.00 | 31.2% |" in text
 
 
+def _write_trace(d, durations):
+    rows, t = [], 0
+    for name, dur in durations:
+        rows.append({"Kernel_Name": name, "Grid_Size_X": 1, "Start_Timestamp": t,
+                     "End_Timestamp": t + dur})
+        t += dur + 500
+    d.mkdir()
+    with open(d / "f_kernel_trace.csv", "w", newline="") as fh:
+        w = csv.DictWriter(fh, fieldnames=list(rows[0]))
+        w.writeheader()
+        w.writerows(rows)
+    with open(d / "f_kernel_stats.csv", "w", newline="") as fh:
+        csv.writer(fh).writerow(["Name", "Calls", "AverageNs", "MinNs", "MaxNs", "Percentage"])
+    return str(d)
+
+
+def _wide(kind: str, resolve: int) -> str:
+    return (f"void (anonymous namespace)::{kind}_wide_kernel<((anonymous namespace)::Resolve)"
+            f"{resolve}, {8 if kind == 'gateup' else 3}>((anonymous namespace)::SwigluArgs)")
+
+
+def test_trace_summary_knows_the_kernels_of_prompts(tmp_path):
+    """A forward that starts with a prompt's router, and the many-row K3
+    kernels: in the library table and as K3 rows of their own."""
+    many = "void (anonymous namespace)::router_logits_many_kernel(unsigned short const*)"
+    text = pmc.summarize_trace(_write_trace(tmp_path / "t", [
+        ("void encode_setup_kernel(int)", 50_000), (many, 20_000),
+        (_wide("gateup", 1), 200_000), (_wide("down", 1), 100_000),
+        (_wide("gateup", 0), 30_000), (_wide("down", 0), 20_000),
+        (_name("gateup", 2), 55_000), (_name("down", 2), 33_000),
+        ("void (anonymous namespace)::router_logits_kernel<4>(int)", 6_000)]), split=False)
+    assert "encode_setup_kernel" not in text
+    library = text.split("## Kernels of libspecfit_amd")[1].split("##")[0]
+    for name in ("router_logits_many_kernel", "gateup_wide_kernel", "down_wide_kernel"):
+        assert name in library
+    rows = {l.split("|")[1].strip(): [c.strip() for c in l.split("|")[2:-1]]
+            for l in text.split("## K3 launches")[1].splitlines() if l.startswith("| all")}
+    assert rows["all, slot table, many rows"] == ["1", "200.00", "100.00", "300.00", "n/a", "n/a"]
+    assert rows["all, many rows"] == ["1", "30.00", "20.00", "50.00", "n/a", "n/a"]
+    assert rows["all"][:4] == ["1", "55.00", "33.00", "88.00"]
+
+
+def test_traffic_summary_names_the_dispatches_it_leaves_out(tmp_path):
+    cal = (CAL, 1 << 20, (256 << 20) / 1024)
+    pair = [(_name(k, 2), _grid(k, 2, 3), 1000.0) for k in ("gateup", "down")]
+    run = lambda name, counter, extra: _counter_dir(tmp_path, name, counter, pair + extra + [cal])
+    plain = pmc.summarize(run("f", "FETCH_SIZE", []), run("w", "WRITE_SIZE", []))
+    assert "many-row" not in plain
+    wide = [(_wide("gateup", 0), 8 * 48 * pmc.THREADS, 5.0), (_wide("down", 0), 8 * 64 * pmc.THREADS, 5.0)]
+    text = pmc.summarize(run("f2", "FETCH_SIZE", wide), run("w2", "WRITE_SIZE", wide))
+    assert "2 dispatches of the many-row K3 kernels" in text
+    ratio = lambda t: next(l for l in t.splitlines() if l.startswith("traffic_ratio_in_step"))
+    assert ratio(text) == ratio(plain)
+
+
 def test_bench_helpers():
     assert bench._union_length([(0, 2), (1, 3), (5, 6)]) == 4
     assert bench._union_length([]) == 0
