@@ -327,8 +327,9 @@ struct TiledArgs {
 // p = exp2(s c - m c) is one fused multiply-add per score, but it subtracts
 // the rounded m c from the exact s c.  Up to this |m c| the difference at the
 // row's maximum is at most 2^-13, far below the rounding of P to bf16 (2^-9);
-// at 2^31 it would be 128, and the row's sum 0 or infinite.  A wavefront with
-// a row past it subtracts before it scales.
+// at 2^31 it would be 128, and the row's sum 0 or infinite.  Rows past it
+// subtract before they scale (a wavefront with such a row runs the subtraction,
+// of 0 for its other rows).
 constexpr float kFusedMax = 4096.f;
 
 // A wavefront multiplies V by what the bf16 rounding of P left in the first
@@ -646,13 +647,14 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
         m = mnew;
       }
       float base = m == -INFINITY ? 0.f : -(m * c);
-      if (__any(fabsf(base) > kFusedMax)) {
-        const float top = m == -INFINITY ? 0.f : m;
+      const bool large = fabsf(base) > kFusedMax;
+      if (__any(large)) {
+        const float top = large ? m : 0.f;
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
           for (int i = 0; i < 16; ++i) s[kt][i] -= top;
-        base = 0.f;
+        if (large) base = 0.f;
       }
       float sum[2] = {0.f, 0.f};
 #pragma unroll

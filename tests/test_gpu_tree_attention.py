@@ -325,6 +325,19 @@ def test_call_without_scratch_uses_the_best_unsplit_form(device):
     assert whole < 7 * split, (whole, split)
 
 
+@pytest.mark.parametrize("Q,S", [(61, 1085), (1024, 1024)])
+def test_a_row_does_not_depend_on_the_scores_of_others(device, Q, S):
+    Hq, Hkv, D = 8, 2, 128
+    g = torch.Generator().manual_seed(Q)
+    q, k, v = (_rand((1, h, n, D), device, g) for h, n in ((Hq, Q), (Hkv, S), (Hkv, S)))
+    plain = ops.tree_attention(q, k, v, None, 0.09)
+    q[0, ::2, ::3] *= 1e6
+    mixed = ops.tree_attention(q, k, v, None, 0.09)
+    rows = torch.ones((Q, Hq), dtype=torch.bool, device=device)
+    rows[::3, ::2] = False
+    assert torch.equal(mixed[0][rows], plain[0][rows])
+
+
 def test_argument_errors(device):
     q = torch.zeros((1, 4, 2, 8), dtype=torch.bfloat16, device=device)
     k = torch.zeros((1, 3, 5, 8), dtype=torch.bfloat16, device=device)
