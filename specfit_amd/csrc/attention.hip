@@ -341,6 +341,9 @@ constexpr float kFusedMax = 4096.f;
 // device time of the last three: 4096-token prompt 1.97 / 2.05 / 1.84 / 1.77,
 // 174 / 189 / 204 us; 512 tokens after 3000: 2.17 / 2.23 / 2.09 / 1.95, 55 /
 // 57 / 60 us; 61-node tree, 1085 keys: 2.09 / 2.11 / 1.91 / 1.91, 16 us each.
+// (Every 6th: 2.17 for 2000 tokens after 2096, where eight maxima have 2.16
+// and every 4th 2.12.)  A tile with an infinite value or NaN goes without: the
+// rest may be 0 or negative where its key has a weight.
 constexpr int kRestTurns = 4;
 
 // Rows padded so the fragment reads spread over the banks: 16 B for the
@@ -363,6 +366,24 @@ constexpr int tiled_lds_bytes() {
 
 __device__ __forceinline__ sf_f32x16 mfma_32(sf_bf16x8 a, sf_bf16x8 b, sf_f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Whether any of a thread's pieces of a value tile holds infinity or NaN: then
+// their sum is not finite (nor is that of finite values past fp32's range,
+// which may go without the rest too).
+template <int N>
+__device__ __forceinline__ bool has_nonfinite(const sf_u32x4 (&v)[N]) {
+  const sf_bf16x2 one = __builtin_bit_cast(sf_bf16x2, 0x3f803f80u);
+  float sum[2] = {0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t w = v[j][i];
+      sum[i & 1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(sf_bf16x2, w), one,
+                                                   sum[i & 1], false);
+    }
+  return !(fabsf(sum[0]) < INFINITY && fabsf(sum[1]) < INFINITY);
 }
 
 // 16-byte load, explicitly from global memory (a flat load would also hold
@@ -488,6 +509,8 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
   constexpr int kLoads = kRowLanes / WR;    // pieces of a 64-row tile per thread
   using L = TileLds<D>;
   __shared__ __attribute__((aligned(16))) char lds[tiled_lds_bytes<D, WR>()];
+  // WR = 4: what each wavefront found in its part of the value tile.
+  __shared__ __attribute__((aligned(16))) int nonfinite[2][kTileWaves];
   const int lane = threadIdx.x & (SF_WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SF_WAVE);
   const int kg = wave / WR;
@@ -589,6 +612,11 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
       *reinterpret_cast<sf_u32x4*>(ktile + r * L::krow + 16 * ld_col) = kr[j];
       *reinterpret_cast<sf_u32x4*>(vtile + r * L::vrow + 16 * ld_col) = vr[j];
     }
+    bool rest = turn % kRestTurns == 0;
+    if (rest) {
+      rest = !__any(has_nonfinite(vr));
+      if (WR == 4 && lane == 0) nonfinite[buf][wave] = !rest;
+    }
     uint32_t mc[8];
     if (MASK) {
 #pragma unroll
@@ -668,7 +696,13 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
       const char* vlane = vtile + (4 * hf + ((lane & 15) >> 2)) * L::vrow +
                           32 * ((lane >> 4) & 1) + 8 * (lane & 3);
       add_values<D, false>(s, vlane, acc);
-      if (turn % kRestTurns == 0) add_values<D, true>(s, vlane, acc);
+      if (turn % kRestTurns == 0) {
+        if (WR == 4) {
+          const int4 bad = *reinterpret_cast<const int4*>(nonfinite[buf]);
+          rest = !__builtin_amdgcn_readfirstlane(bad.x | bad.y | bad.z | bad.w);
+        }
+        if (rest) add_values<D, true>(s, vlane, acc);
+      }
     }
     if (WR != 4) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // tile reused
   }

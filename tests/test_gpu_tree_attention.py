@@ -338,6 +338,53 @@ def test_a_row_does_not_depend_on_the_scores_of_others(device, Q, S):
     assert torch.equal(mixed[0][rows], plain[0][rows])
 
 
+@pytest.mark.parametrize("Q,S,masked", [(1, 4096, False), (61, 1085, True), (200, 200, False),
+                                        (1024, 1024, False), (700, 900, True)])
+def test_infinities_and_nan(device, Q, S, masked):
+    """An infinite value stays infinite for the rows that admit its key; NaN
+    and infinite scores touch their own rows only (zeros, as in the loop form,
+    whose sum is NaN there too)."""
+    Hq, Hkv, D = 8, 2, 128
+    g = torch.Generator().manual_seed(Q)
+    q, k, v = (_rand((1, h, n, D), device, g) for h, n in ((Hq, Q), (Hkv, S), (Hkv, S)))
+    mask = torch.ones((1, 1, Q, S), dtype=torch.bool, device=device) if masked else None
+    clean = ops.tree_attention(q, k, v, mask, 0.09)
+    for key in (0, 63, S // 2, S - Q):
+        for value in (math.inf, -math.inf):
+            bad = v.clone()
+            bad[0, 1, key, 7] = value
+            out = ops.tree_attention(q, k, bad, mask, 0.09)
+            first = 0 if masked else max(0, key - (S - Q))  # rows that admit the key
+            assert bool((out[0, first:, Hq // 2:, 7] == value).all()), (key, value)
+            keep = torch.ones_like(out, dtype=torch.bool)
+            keep[0, :, Hq // 2:, 7] = False  # equal but for the rest of P's rounding
+            err = (out.float() - clean.float())[keep].abs().max()
+            assert err.item() <= 1e-2 * clean.float().abs().max().item()
+    for value in (math.nan, math.inf):
+        bad = q.clone()
+        bad[0, 3, Q // 2, 5] = value
+        out = ops.tree_attention(bad, k, v, mask, 0.09)
+        rows = torch.ones((Q, Hq), dtype=torch.bool, device=device)
+        rows[Q // 2, 3] = False
+        assert torch.equal(out[0][rows], clean[0][rows])
+        assert not out[0, Q // 2, 3].any()
+    # A key of -inf in one element: weight 0 for rows with a positive query
+    # there (the row is that of the other keys), zeros for the others.
+    bad = k.clone()
+    bad[0, 0, S - Q, 9] = -math.inf
+    out = ops.tree_attention(q, bad, v, mask, 0.09)
+    without = torch.ones((1, 1, Q, S), dtype=torch.bool, device=device) if masked else (
+        torch.arange(S, device=device) <= S - Q + torch.arange(Q, device=device)[:, None])[None, None]
+    without = without.clone()
+    without[..., S - Q] = False
+    ref = _reference(q, k, v, without, 0.09)
+    positive = (q[0, :Hq // 2, :, 9] > 0).T  # [Q, heads of KV head 0]
+    got, want = out[0, :, :Hq // 2][positive], ref[0, :, :Hq // 2][positive]
+    _check(got, want)
+    negative = (q[0, :Hq // 2, :, 9] < 0).T
+    assert not out[0, :, :Hq // 2][negative].any()
+
+
 def test_argument_errors(device):
     q = torch.zeros((1, 4, 2, 8), dtype=torch.bfloat16, device=device)
     k = torch.zeros((1, 3, 5, 8), dtype=torch.bfloat16, device=device)
