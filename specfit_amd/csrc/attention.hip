@@ -584,12 +584,15 @@ __global__ __launch_bounds__(kTileThreads, WR == 4 ? 2 : 1) void tree_attention_
 #pragma unroll
       for (int j = 0; j < kLoads; ++j) vr[j] = ld16(vp + j * kRowsPerLoad * a.v_tok, v_off);
     } else {
-      // Rows past the end repeat the last key: finite values that meet p = 0.
+      // Rows past the end: the last key's score, masked, and values of 0 (an
+      // infinite last value would meet p = 0).
 #pragma unroll
       for (int j = 0; j < kLoads; ++j) {
-        const int64_t key = min(kb + j * kRowsPerLoad + ld_row, a.S - 1);
+        const int at = kb + j * kRowsPerLoad + ld_row;
+        const int64_t key = min(at, a.S - 1);
         kr[j] = ld16(kh + key * a.k_tok + 8 * ld_col);
-        vr[j] = ld16(vh + key * a.v_tok + 8 * ld_col);
+        vr[j] = sf_u32x4(0u);
+        if (at < a.S) vr[j] = ld16(vh + key * a.v_tok + 8 * ld_col);
       }
     }
     if (MASK) {

@@ -339,7 +339,7 @@ def test_a_row_does_not_depend_on_the_scores_of_others(device, Q, S):
 
 
 @pytest.mark.parametrize("Q,S,masked", [(1, 4096, False), (61, 1085, True), (200, 200, False),
-                                        (1024, 1024, False), (700, 900, True)])
+                                        (1024, 1024, False), (700, 900, True), (5, 1056, False)])
 def test_infinities_and_nan(device, Q, S, masked):
     """An infinite value stays infinite for the rows that admit its key; NaN
     and infinite scores touch their own rows only (zeros, as in the loop form,
@@ -349,7 +349,7 @@ def test_infinities_and_nan(device, Q, S, masked):
     q, k, v = (_rand((1, h, n, D), device, g) for h, n in ((Hq, Q), (Hkv, S), (Hkv, S)))
     mask = torch.ones((1, 1, Q, S), dtype=torch.bool, device=device) if masked else None
     clean = ops.tree_attention(q, k, v, mask, 0.09)
-    for key in (0, 63, S // 2, S - Q):
+    for key in (0, 63, S // 2, S - Q, S - 1):
         for value in (math.inf, -math.inf):
             bad = v.clone()
             bad[0, 1, key, 7] = value
