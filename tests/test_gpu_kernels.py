@@ -402,6 +402,76 @@ def test_many_row_kernels_match_the_streaming_split(device, H, I):
         assert torch.equal(y[lo:lo + 128], ops.expert_swiglu(x[lo:lo + 128], slots[2], H, I))
 
 
+@pytest.mark.parametrize("H,I,counts", [
+    (2048, 768, [530, 257, 161, 160, 129, 97, 96, 65, 64, 33, 32, 17, 16, 1, 0]),
+    (4096, 1536, [300, 130, 100, 70, 40, 20, 3])])
+def test_many_row_lists_match_the_oracle(device, H, I, counts):
+    """A list launch of mixed row counts (some through the tiled bodies, some
+    through the streaming ones) against the CPU oracle, with and without its
+    intermediate roundings.  Against the rounded one single values move by a
+    bf16 step (2^-7 at most) where fp32 sums in another order round otherwise,
+    and once more in the product with the routing weight; against the unrounded
+    one six roundings of 2^-9 at most (gate, up, silu, their product, the row,
+    the scaled row), 2^-9 times sqrt(6) in the 2-norm, and twice that as the
+    bar, as silu's slope passes gate's on with a factor of up to 1.1."""
+    E, T = len(counts), max(counts)
+    g = torch.Generator("cpu").manual_seed(I)
+    hidden = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    packed = (torch.randn(E, 3 * H * I, generator=g) * 0.02).to(torch.bfloat16)
+    idx = torch.full((T, E), -1, dtype=torch.int64)
+    for e, m in enumerate(counts):
+        idx[torch.randperm(T, generator=g)[:m], e] = e
+    weights = torch.rand(T, E, generator=g).to(torch.bfloat16)
+    h_dev, slots = hidden.to(device), packed.to(device)
+    plan = ops.dispatch(idx.to(device), E)
+    plan.fetch_counts()
+    assert plan.count_list[:E] == counts
+    act = torch.empty((T * E, I), dtype=torch.bfloat16, device=device)
+    rows = torch.zeros((T * E, H), dtype=torch.bfloat16, device=device)
+    listed = [e for e in range(E) if e != 3]  # one expert stays out of the launch
+    ops.grouped_swiglu(h_dev, plan, weights.to(device).reshape(-1), listed, [slots[e] for e in listed],
+                       H, I, act, rows, slot_storage=slots)
+    perm = plan.perm_pos.cpu().long()
+    x, w = oracle.bf16_float(_bits(hidden)), weights.float().reshape(-1).numpy()
+    for e, m in enumerate(counts):
+        lo = plan.offset_list[e]
+        got = oracle.bf16_float(_bits(rows[lo:lo + m]))
+        if e not in listed:
+            assert not got.any()
+        elif m:
+            pos = perm[lo:lo + m].numpy()
+            one = oracle.bf16_float(_bits(packed[e]))
+            ref = oracle.round_bf16(oracle.expert_forward_bf16(x[pos // E], one, H, I) * w[pos][:, None])
+            np.testing.assert_allclose(got, ref, rtol=1.6e-2, atol=1.6e-2 * ref.std())
+            exact = oracle.expert_forward_fp32(x[pos // E], one, H, I) * w[pos][:, None]
+            assert np.linalg.norm(got - exact) <= 2 * 6 ** 0.5 * 2 ** -9 * np.linalg.norm(exact), (e, m)
+
+
+def test_bf16_rounding_of_every_sum(device):
+    """Rounding to bf16 (round to nearest even, NaN quiet) through the combine:
+    every bf16 pattern plus eight others each, among them ties, subnormal sums,
+    overflow, infinities and NaN, against the integer form."""
+    H, K = 2048, 2
+    a = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    rng = np.random.default_rng(4)
+    others = [(a ^ 0x8000) + 1, np.full_like(a, 0x3380), np.full_like(a, 0x7F7F), np.full_like(a, 0x0001),
+              np.full_like(a, 0xFF80), a - (7 << 7), a - (8 << 7) + 1,
+              rng.integers(0, 65536, a.size).astype(np.uint16)]
+    for other in others:
+        T = a.size // H
+        idx = torch.arange(K, device=device).expand(T, K).contiguous()
+        plan = ops.dispatch(idx, K)
+        rows = np.concatenate([a.reshape(T, H), other.reshape(T, H)])  # expert 0's rows, expert 1's
+        out = _bits(ops.combine(_from_bits(rows, device), idx, plan, H, accumulate_fp32=True)).reshape(-1)
+        with np.errstate(all="ignore"):
+            total = (np.float32(0) + oracle.bf16_float(a)) + oracle.bf16_float(other)
+        u = total.view(np.uint32).astype(np.uint64)
+        want = ((u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+        nan = np.isnan(total)
+        np.testing.assert_array_equal(out[~nan], want[~nan])
+        assert ((out[nan] & 0x7FC0) == 0x7FC0).all()
+
+
 def test_many_rows_into_unaligned_output_rows(device):
     """The tiled kernels store 8 bytes at a time; output rows off that
     alignment take the streaming kernels, with the same bits."""
