@@ -122,7 +122,7 @@ int sf_router_topk(const void *hidden, const void *router_weight, int tokens,
  *              device-to-host copy (the reference's one host read of the
  *              routed experts, qwen3_offloaded_experts.py:111-113).  Memory
  *              the device cannot map returns SF_ERR_INVALID_ARGUMENT.
- * One workgroup; any tokens >= 0.
+ * One workgroup for up to 1024 routes, up to 256 above; any tokens >= 0.
  */
 int sf_dispatch(const int64_t *topk_index, int tokens, int top_k,
                 int num_experts, int32_t *counts, int32_t *offsets,
@@ -321,7 +321,10 @@ int sf_expert_decode(const void *record, size_t record_bytes, int64_t n_values,
  * qh = h * G + j (G = q_heads / kv_heads, h the key/value head):
  *   out[qi, qh, :] = sum_s p_s * v[h, s, :],
  *   p = softmax over admitted keys s of scale * (q[qi, qh, :] . k[h, s, :])
- * computed in fp32 and rounded to bf16 once.  Key s is admitted when
+ * with scores and sums in fp32 and the result rounded to bf16 once.  The form
+ * for 16-byte aligned rows, head_dim 64 or 128 and G >= 2 multiplies V by p
+ * rounded to bf16 (relative to the row's running maximum), and by the rest of
+ * that rounding for part of the keys.  Key s is admitted when
  * mask[qi * mask_stride_query + s] != 0; with mask == NULL, when
  * s <= keys - queries + qi (causal, aligned to the end of the keys).  A
  * query with no admitted key gets zeros.

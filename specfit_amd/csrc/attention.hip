@@ -11,13 +11,13 @@
 // gets 0.
 //
 // Head dims 64 and 128 with 2..16 query heads per KV head run the tiled MFMA
-// form below; measured on MI355X at 32 query / 4 KV heads of 128, against the
-// 16-row MFMA form it replaced: a 4096-token prompt 1562 -> 162 us (850
-// TFLOP/s of the causal half), one token over 4096 keys 49 -> 10 us of device
-// time, a 61-node tree over 1085 keys 26 -> 16 us.  What bounds it: prompts,
-// the softmax's vector work next to the matrix work (each SIMD has two
-// wavefronts, which overlap only in part); decoding and trees, latency (the
-// K/V of 1085 keys is 2 MB).
+// form below; device time on MI355X at 32 query / 4 KV heads of 128, against
+// the 16-row MFMA form it replaced: a 4096-token prompt 1565 -> 187 us (735
+// TFLOP/s of the causal half), one token over 4097 keys 49 -> 9.3 us, a 61-node
+// tree over 1085 keys 26 -> 17 us; at 16 / 4 heads of 64: 2048 tokens 106 ->
+// 36 us, 35 -> 8 and 18 -> 9 us.  What bounds it: prompts, the softmax's vector
+// work next to the matrix work (each SIMD has two wavefronts, which overlap
+// only in part); decoding and trees, latency (the K/V of 1085 keys is 2 MB).
 // The loop form covers every other shape: one workgroup per (query, KV head)
 // keeps the G query heads of the group together so each K/V row is read once
 // per query.  Its 8 wavefronts take interleaved 64-key chunks: scores with one
@@ -873,12 +873,17 @@ struct TiledPlan {
 // short calls wait for) and the partial states' way through memory (0.28 ns
 // per row and split, 1 KiB each); a CU runs one WR = 1 workgroup at a time,
 // and WR = 4 workgroups above 1.5 per CU wait for each other.  Measured at 32
-// query / 4 KV heads of 128 (us):
+// query / 4 KV heads of 128 (us; all but the first line before the rest of P,
+// which lengthens every form by 2 - 10%):
 //   1 query, 4097 keys:     82.6 unsplit, 9.0 in 33 splits (WR = 4); 43.7 unsplit (WR = 1)
 //   32 queries, 1056 keys:  21.8 unsplit, 12.2 in 5 (WR = 1); 13.4 WR = 4
 //   61 queries, 1085 keys:  22.0 unsplit, 15.9 in 3, 20.2 in 5 (WR = 1)
 //   129 queries, 8129 keys: 227 unsplit, 46.8 in 11, 54.3 in 32 (WR = 4)
 //   256 queries and keys:   8.8 unsplit (WR = 1), 10.9 (WR = 4), 13.9 in 2
+// Head dim 64 shares these numbers; its steps are shorter, and its plans were
+// only checked against the form before the key splits (16 / 4 heads: 64
+// queries, 4096 keys: 35.7 -> 10.6; 256, 3000: 30.3 -> 16.5; 129, 8129 with a
+// mask: 96.7 -> 27.4).
 // may_split: the caller has scratch for the partial states.
 TiledPlan tiled_plan(int queries, int keys, int kv_heads, int G, bool mask, bool may_split) {
   const int64_t rows = static_cast<int64_t>(queries) * G;

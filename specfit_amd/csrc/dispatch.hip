@@ -15,11 +15,11 @@
 // Every workgroup counts all routes itself, those before its span and the
 // rest apart: that gives it the expert offsets and the starting ranks of its
 // span without scratch memory, a second launch or waiting for another
-// workgroup.  Up to kMaxSpans spans the extra reads stay below 8 B * N *
-// kMaxSpans (34 MB of L2 hits for the 16384 routes of a 2048-token prompt,
-// 16 spans), and past that a span holds several chunks.  One workgroup with a
-// ballot round per distinct id took 87 us for those 16384 routes and left
-// 255 CUs idle.
+// workgroup.  The extra reads are 8 B * N per span (2.1 MB of L2 hits for the
+// 16384 routes of a 2048-token prompt, 16 spans), at most kMaxSpans of them;
+// past that a span holds several chunks.  One workgroup with a ballot round per
+// distinct id took 86 us for those 16384 routes and left 255 CUs idle; 16 take
+// 7.1 us (E = 128, uniform routing; 8.6 Zipf).  512 routes: 6.0 -> 3.9 us.
 #include "sf_common.h"
 
 namespace {

@@ -674,8 +674,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(
 }
 
 // -------------------------------------------------------- many-row experts --
-// Launches whose experts average many rows (a prompt: about T K / E rows per
-// expert) take a tiled GEMM instead of the streaming split above, which
+// Launches with enough experts of many rows (a prompt: about T K / E rows per
+// expert; the rule is wide_launch's) take a tiled GEMM instead of the streaming split above, which
 // re-reads its token rows for every 16 activation (32 output) columns and
 // feeds the matrix cores 32 x 32 per wavefront: at 128 rows per expert it was
 // bound by those re-reads (L2), not by the weights.
