@@ -855,10 +855,12 @@ bool scale_ok(float scale) {
 }
 
 // Shapes of the tiled form: head dim 64 or 128, 2..16 query heads per KV head
-// (powers of two).
-bool tiled_shape(int queries, int G, int head_dim) {
+// (powers of two), row and key numbers that stay in 32 bits (a plan's splits
+// reach up to kMaxSplits steps past the last key).
+bool tiled_shape(int queries, int keys, int G, int head_dim) {
   return (head_dim == 64 || head_dim == 128) && G >= 2 && G <= 16 && (G & (G - 1)) == 0 &&
-         static_cast<int64_t>(queries) * G <= 0x3fffffff;
+         static_cast<int64_t>(queries) * G <= 0x3fffffff &&
+         keys <= 0x7fffffff - 4 * kMaxSplits * kTileKeys * kTileWaves;
 }
 
 // Row groups (WR) and key splits of a call.
@@ -1048,7 +1050,7 @@ int attention_call(const void* q, int64_t q_stride_token, int64_t q_stride_head,
   a.out = static_cast<uint16_t*>(out);
   // The tiled form: 16-byte aligned query / key / value rows (8-element
   // strides) and a scale its log2 units can hold.
-  const bool tiled = tiled_shape(queries, G, head_dim) && aligned(q, 16) && aligned(v, 16) &&
+  const bool tiled = tiled_shape(queries, keys, G, head_dim) && aligned(q, 16) && aligned(v, 16) &&
                      aligned(out, 8) && q_stride_token % 8 == 0 && q_stride_head % 8 == 0 &&
                      v_stride_token % 8 == 0 && v_stride_head % 8 == 0 &&
                      k_stride_token < (1 << 24) && v_stride_token < (1 << 24) &&
@@ -1083,7 +1085,7 @@ extern "C" int64_t sf_tree_attention_workspace(int queries, int keys, int q_head
                                                int head_dim, int masked) {
   if (queries < 1 || keys < 1 || kv_heads < 1 || q_heads < kv_heads || q_heads % kv_heads) return 0;
   const int G = q_heads / kv_heads;
-  if (!tiled_shape(queries, G, head_dim)) return 0;
+  if (!tiled_shape(queries, keys, G, head_dim)) return 0;
   return tiled_workspace(tiled_plan(queries, keys, kv_heads, G, masked != 0, true), queries,
                          q_heads, head_dim);
 }

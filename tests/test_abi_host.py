@@ -160,3 +160,16 @@ def test_attention_scratch_is_only_for_calls_that_split():
             assert work(queries, keys, q_heads, kv_heads, 128, masked) == 0, (q_heads, kv_heads)
     for q_heads, kv_heads in [(8, 4), (16, 4), (32, 4), (64, 4)]:
         assert work(1, 4096, q_heads, kv_heads, 128, 0) > 0
+
+
+def test_attention_key_numbers_stay_in_32_bits():
+    """Up to the last size that the split form takes, its splits cover the
+    keys and end within 32 bits; past it there is no split (nor scratch)."""
+    work = _native.lib().sf_tree_attention_workspace
+    last = (1 << 31) - 1 - 4 * 64 * 256
+    for keys in (1 << 30, 3 << 29, last):
+        for masked in (0, 1):
+            splits = work(1, keys, 32, 4, 128, masked) // (32 * 130 * 4)
+            assert 2 <= splits <= 64
+    for keys in (last + 1, (1 << 31) - 257, (1 << 31) - 1):
+        assert work(1, keys, 32, 4, 128, 0) == 0, keys
